@@ -106,7 +106,11 @@ extern "C" {
 #define SN_PRECISION_BF16 2u
 /* Kernel selection, the role of the reference's MatmulKernel
  * (device.rs:38-67; public field Gpu::matmul_kernel, device.rs:144):
- *   SN_KERNEL_MFMA_F32  fp32 matrix-core GEMM (default; the role of Blocked)
+ *   SN_KERNEL_MFMA_F32  fp32 matrix-core GEMM (default; the role of Blocked);
+ *                       tiled products split each fp32 operand exactly into
+ *                       three bf16 parts and accumulate their products in
+ *                       fp32 (nearer the 64-bit result than fp32 products
+ *                       added one by one)
  *   SN_KERNEL_MFMA_BF16 inputs rounded to bf16 (nearest-even), fp32
  *                       accumulation (the role of TensorCore's TF32)
  *   SN_KERNEL_SIMPLE    one thread per output, k summed in order with
@@ -242,9 +246,9 @@ int sn_matmul_bias(sn_context *context, const sn_matmul_spec *spec, const float 
  * The right operand must be stored row-major ([inner, cols], spec->right ==
  * SN_ROW_MAJOR) and the spec unbatched (SN_ERR_UNSUPPORTED otherwise);
  * sums_len must equal spec->cols (SN_ERR_LENGTH_MISMATCH); sums must not
- * overlap the output or the operands (SN_ERR_ALIASING). fp32 products the
- * direct-to-LDS kernel serves add the column sums while the right operand's
- * tiles pass through LDS, and bf16 products the 256 x 256 kernel serves while
+ * overlap the output or the operands (SN_ERR_ALIASING). Aligned fp32 products
+ * add the column sums while the right operand's tiles pass through the
+ * registers, and bf16 products the 256 x 256 kernel serves while
  * its fp32 values pass through the registers before rounding: the first tile
  * row of each K slice sums them (or, where the right operand is the one
  * staged as bf16, the staging pass sums each 64 k as it reads them), in a
@@ -471,8 +475,8 @@ int sn_matmul_noalloc(const sn_matmul_spec *spec, const float *left, size_t left
 #define SN_PATH_REFERENCE_ORDER 1u /* SN_KERNEL_SIMPLE: one thread per output */
 #define SN_PATH_FEW_ROWS 2u        /* decode GEMV: at most 16 rows, right operand row-major */
 #define SN_PATH_FEW_ROWS_NT 3u     /* at most 4 rows against a right operand stored [cols][inner] */
-#define SN_PATH_F32_DIRECT 4u      /* fp32 tiles, operands loaded straight into LDS */
-#define SN_PATH_F32_REGISTER 5u    /* fp32 tiles, operands staged through registers (unaligned) */
+#define SN_PATH_F32_DIRECT 4u      /* fp32 tiles, operands that 16-byte loads serve */
+#define SN_PATH_F32_REGISTER 5u    /* fp32 tiles, other operands (unaligned) */
 #define SN_PATH_BF16_STAGED 6u     /* bf16: both operands first rounded into the workspace */
 #define SN_PATH_BF16_DIRECT 7u     /* bf16: fp32 LDS stages rounded per fragment */
 #define SN_PATH_BF16_REGISTER 8u   /* bf16: register-staged (unaligned) operands */

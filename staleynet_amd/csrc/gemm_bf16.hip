@@ -5,7 +5,7 @@
 // into LDS, products summed in fp32. Tolerance 2e-2 in the reference's metric.
 //
 // The operands stay fp32 in HBM (the boundary hands over f32 tensors), so the
-// global loads, schedule, split-K and masks are those of gemm_mfma.hip. The
+// tiles, grid, split-K and masks are the fp32 engine's (gemm_f32.h). The
 // LDS stage is bf16 in [BK/8 k-octets][ROWS + PAD][8 bf16] 16-byte slots;
 // each loader writes a group of four k as one 8-byte half slot, and PAD is
 // chosen per loader layout so the 16 lanes of a b64 write phase hit

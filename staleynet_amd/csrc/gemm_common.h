@@ -1,7 +1,6 @@
 // Pieces shared by the fp32 and bf16 matrix-core GEMMs: buffer addressing,
 // kernel arguments, the LDS geometry, the operand loaders, the tile
-// schedule, split-K planning and the reference's combine. See
-// gemm_mfma.hip for the design these serve.
+// map, split-K planning and the reference's combine.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -127,15 +126,6 @@ struct Tile {
     static_assert(BK == 32, "the loaders' lane mappings assume 8 k-groups of 4 per tile");
 };
 
-// fp32 LDS geometry of one operand tile: BK/4 planes (k-groups) of ROWS + 1
-// 16-byte slots; slot (g, r) holds k = 4g .. 4g+3 of row r.
-template <int ROWS, int BK>
-struct Planes {
-    static constexpr int PLANE = ROWS + 1;
-    static constexpr int GROUPS = BK / 4;
-    static constexpr int SLOTS = GROUPS * PLANE;
-};
-
 // bf16 LDS geometry: BK/8 planes (k-octets) of ROWS + PAD 16-byte slots;
 // slot (o, r) holds k = 8o .. 8o+7 of row r as bf16. A loader writes each
 // group of four k as one 8-byte half-slot. PAD is chosen per loader so that
@@ -150,7 +140,7 @@ struct OctetPlanes {
 // Operand loaders. Each stages a ROWS x BK tile of one operand per K-step
 // through registers into LDS. `init` runs once per tile, `load` issues the
 // global reads for the K-step starting at k0 (reading 0 outside the matrix),
-// `store` writes one fp32 LDS stage, `store_bf16` one bf16 stage.
+// `store_bf16` writes one bf16 LDS stage.
 //
 // K-contiguous operands (element (r, k) at base[r * ld + k]): vector v of a
 // thread is row idx / 8, k-group idx % 8 (idx = tid + v * THREADS), so the 8
@@ -164,7 +154,6 @@ struct OctetPlanes {
 // buffer offsets: one bounds check per element.
 template <int ROWS, int BK, int THREADS>
 struct KContiguousScalarLoader {
-    using P = Planes<ROWS, BK>;
     static constexpr int GROUPS = BK / 4;
     static constexpr int TOTAL = ROWS * GROUPS;
     static constexpr int PER_THREAD = (TOTAL + THREADS - 1) / THREADS;
@@ -203,17 +192,6 @@ struct KContiguousScalarLoader {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (gk + e > gr + offset) reg[v][e] = 0.f;
-        }
-    }
-
-    __device__ __forceinline__ void store(float* lds, int tid) const {
-#pragma unroll
-        for (int v = 0; v < PER_THREAD; ++v) {
-            const int idx = tid + v * THREADS;
-            if (TOTAL % THREADS == 0 || idx < TOTAL) {
-                const int slot = (idx % GROUPS) * P::PLANE + idx / GROUPS;
-                *reinterpret_cast<f32x4*>(lds + 4 * slot) = reg[v];
-            }
         }
     }
 
@@ -263,7 +241,6 @@ struct KContiguousBufferLoader : KContiguousScalarLoader<ROWS, BK, THREADS> {
 
 template <int ROWS, int BK, int THREADS>
 struct RowContiguousScalarLoader {
-    using P = Planes<ROWS, BK>;
     static constexpr int GROUPS = BK / 4;
     static constexpr int TOTAL = GROUPS * (ROWS / 4);
     static constexpr int PER_THREAD = (TOTAL + THREADS - 1) / THREADS;
@@ -308,21 +285,6 @@ struct RowContiguousScalarLoader {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (gr + e > gk + offset) reg[v][kk][e] = 0.f;
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(float* lds, int tid) const {
-#pragma unroll
-        for (int v = 0; v < PER_THREAD; ++v) {
-            const int idx = tid + v * THREADS;
-            if (TOTAL % THREADS == 0 || idx < TOTAL) {
-                const int first = (idx % GROUPS) * P::PLANE + (idx / GROUPS) * 4;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    f32x4 t = {reg[v][0][e], reg[v][1][e], reg[v][2][e], reg[v][3][e]};
-                    *reinterpret_cast<f32x4*>(lds + 4 * (first + e)) = t;
-                }
             }
         }
     }
@@ -703,7 +665,10 @@ struct Plan {
 // bf16 pairs).
 struct SplitCost {
     int workgroups_per_cu = 2;
-    double flops_per_cu = 522e9;  // fp32 matrix cores at about 85 % of 157.3 TFLOP/s / 256 CUs
+    // fp32: the split counts below were measured at this rate and are kept
+    // (plans are part of what callers see); the split engine runs at about
+    // 1.4 times it.
+    double flops_per_cu = 522e9;
     int k_per_index = 1;
 };
 
@@ -766,6 +731,17 @@ Plan plan_for(const Problem& p, const Env& env, const SplitCost& cost = SplitCos
     return plan;
 }
 
+// Unsplit products with at most 128 inner elements write as many output bytes
+// as they read: their outputs, and the zero tiles of a causal output mask,
+// stream out. Measured on 192 x 2048 x 2048 x 64 attention scores and dP
+// products, dense: 1.38-1.44 -> 1.25 ms and 1.31-1.32 -> 1.17-1.19 ms; causal:
+// 0.91 -> 0.81 ms and 0.88 -> 0.76 ms (fp32 instruction). At K = 768 (the
+// Linear products) streaming stores changed nothing beyond noise.
+constexpr int64_t kStreamingMaxK = 128;
+inline bool streams_output(const Problem& p, const Plan& plan) {
+    return (p.mask == SN_MASK_NONE || p.mask == SN_MASK_CAUSAL_OUTPUT) && plan.splits == 1 && p.k <= kStreamingMaxK;
+}
+
 template <class T>
 LaunchShape tiled_shape(const Problem& p, const Plan& plan, uint32_t path) {
     return tiled_shape<T>(p, plan.tiles_m, plan.tiles_n, plan.splits, plan.k_per_split, path);
@@ -802,12 +778,7 @@ Args make_args(const Problem& p, const Env& env, const Plan& plan) {
     return args;
 }
 
-// The direct-to-LDS fp32 kernel (gemm_dma.hip): whether it serves `p`
-// (aligned operands), its launch shape and its launcher.
-bool dma_applies(const Problem& p, const Env& env);
-LaunchShape describe_f32_dma(const Problem& p, const Env& env);
-hipError_t launch_gemm_f32_dma(const Problem& p, const Env& env, hipStream_t stream);
-// The bf16 variant of the direct-to-LDS kernel: whether it serves `p`, its
+// The direct-to-LDS bf16 kernel (gemm_dma.hip): whether it serves `p`, its
 // launch shape (with the split-K workspace it uses) and its launcher.
 bool bf16_dma_applies(const Problem& p, const Env& env);
 LaunchShape describe_bf16_dma(const Problem& p, const Env& env);
@@ -818,8 +789,8 @@ hipError_t launch_gemm_bf16_dma(const Problem& p, const Env& env, hipStream_t st
 bool bf16_wide_applies(const Problem& p, const Env& env);
 LaunchShape describe_bf16_wide(const Problem& p, const Env& env);
 hipError_t launch_gemm_bf16_wide(const Problem& p, const Env& env, hipStream_t stream);
-// The fp32 direct-to-LDS product that also adds the right operand's column
-// sums into p.column_sums (gemm_dma.hip): whether it serves `p` (batch 1,
+// The fp32 product that also adds the right operand's column sums into
+// p.column_sums (gemm_f32.hip): whether it serves `p` (batch 1,
 // unmasked, no bias, right operand row-contiguous, aligned), its launch shape
 // (workspace: the product's partial sums and N per K slice) and launcher.
 bool f32_column_sums_applies(const Problem& p, const Env& env);
@@ -840,7 +811,7 @@ LaunchShape describe_bf16_staged(const Problem& p, const Env& env);
 hipError_t launch_gemm_bf16_staged(const Problem& p, const Env& env, hipStream_t stream);
 
 // Adds the split-K partial sums in split order and applies the combine
-// (defined in gemm_mfma.hip).
+// (defined in gemm_f32.hip).
 hipError_t launch_splitk_reduce(const Problem& p, const Env& env, int splits, hipStream_t stream);
 
 }  // namespace gemm

@@ -33,7 +33,8 @@ struct Problem {
     const float* bias = nullptr;
     // Linear's bias gradient, fused into the weight-gradient product: sums
     // [c] += the sum over K of the right operand's column c (stored row-major
-    // [K][N]). Only for the fp32 direct-to-LDS kernel, batch 1, unmasked.
+    // [K][N]). Only where the fp32 tile engine or the bf16 256 x 256 kernel
+    // takes it (column_sums_fusion): batch 1, unmasked.
     float* column_sums = nullptr;
 };
 
@@ -238,8 +239,7 @@ hipError_t launch_column_sums_finish(const float* partial, int64_t slices, int64
 
 // The weight-gradient product with the bias gradient (sn_matmul_column_sums):
 // p.column_sums[c] += the sum over K of the right operand's column c, beside
-// the product. Fused into the fp32 direct-to-LDS kernel or the bf16 wide
-// kernel where that serves `p` (column_sums_fusion), else the product and
+// the product. Fused into the fp32 tile engine or the bf16 wide kernel where that serves `p` (column_sums_fusion), else the product and
 // then launch_column_sums; the workspace bytes are then the larger of the
 // two steps'.
 enum class ColumnSumsFusion { None, F32Direct, Bf16Wide };
