@@ -694,6 +694,7 @@ int causal_attention_call(sn_context* ctx, const sn_attention_shape* shape, cons
     args.workspace_bytes = ctx->env.workspace_bytes;
     args.counters = ctx->env.counters;
     args.counter_count = ctx->env.counter_count;
+    args.cu_count = ctx->env.cu_count;
     if (!sn::causal_attention_supported(args)) return SN_ERR_UNSUPPORTED;
     hipError_t err = hipSetDevice(ctx->device);
     if (err == hipSuccess) err = sn::launch_causal_attention(args, ctx->stream);

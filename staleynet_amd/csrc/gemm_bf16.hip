@@ -18,7 +18,6 @@ namespace sn {
 namespace gemm {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 template <class T, class LA, class LB>
 __device__ __forceinline__ void multiply_tile_bf16(const uint16_t* __restrict__ lds_a,

@@ -30,7 +30,6 @@ namespace sn {
 namespace gemm {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 using WideTile = Tile<256, 256, 32, 4, 2>;
 

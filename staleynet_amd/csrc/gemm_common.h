@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "gemm_internal.h"
+#include "split_bf16.h"
 #include "staleynet_gemm.h"
 
 namespace sn {
@@ -74,16 +75,6 @@ __device__ __forceinline__ void buffer_store4_coherent(__amdgpu_buffer_rsrc_t rs
 }
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// Two floats -> two bf16 in one 32-bit word (element 0 in the low half):
-// gfx950's v_cvt_pk_bf16_f32, which rounds by the MODE register's f32
-// rounding mode (round to nearest, ties to even, by default) and keeps NaN a
-// quiet NaN. One instruction per pair instead of a shift/add/compare
-// sequence per element.
-__device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
-}
 
 // Four floats as four bf16 packed into 8 bytes, element 0 in the low half.
 __device__ __forceinline__ u32x2 pack_bf16(f32x4 x) {

@@ -43,7 +43,6 @@ namespace gemm {
 namespace {
 
 typedef __attribute__((address_space(3))) void* lds_void;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
 // Eight floats rounded to bf16 (four v_cvt_pk_bf16_f32).

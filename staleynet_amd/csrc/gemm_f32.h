@@ -69,10 +69,6 @@
 namespace sn {
 namespace gemm {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int kParts = 3;  // hi, mid, lo
-
 // How an operand is loaded.
 //  kLoadVector: 16-byte buffer loads; the contiguous dimension, leading
 //    dimension and base are multiples of 4 floats, so a vector is inside the
@@ -84,25 +80,6 @@ constexpr int kParts = 3;  // hi, mid, lo
 constexpr int kLoadVector = 0;
 constexpr int kLoadDword = 1;
 constexpr int kLoadPointer = 2;
-
-// One third of the split of a pair of values: piece 0 takes hi and leaves the
-// rests in x0 and x1, piece 1 takes mid, piece 2 lo. `upper` is 0xffff0000 in
-// a vector register (v_and with a literal runs at half the rate).
-__device__ __forceinline__ void split_piece(int piece, float& x0, float& x1, uint32_t upper, uint32_t& hi,
-                                            uint32_t& mid, uint32_t& lo) {
-    if (piece == 0) {
-        const uint32_t b0 = __builtin_bit_cast(uint32_t, x0), b1 = __builtin_bit_cast(uint32_t, x1);
-        hi = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-        x0 = x0 - __builtin_bit_cast(float, b0 & upper);
-        x1 = x1 - __builtin_bit_cast(float, b1 & upper);
-    } else if (piece == 1) {
-        mid = pack2_bf16(x0, x1);
-        x0 = x0 - __builtin_bit_cast(float, mid << 16);
-    } else {
-        x1 = x1 - __builtin_bit_cast(float, mid & upper);
-        lo = pack2_bf16(x0, x1);
-    }
-}
 
 // A thread index the compiler cannot trace, so that what is derived from it
 // on a rare path is formed there and not held in registers across the loop.
@@ -320,7 +297,7 @@ struct SplitEngine {
                                          SplitLoaderR<T::BN, T::THREADS, PAIR_N, MODE>>::type;
     using SA = SplitStage<T::BM>;
     using SB = SplitStage<T::BN>;
-    static constexpr int MFMAS = 6 * T::FM * T::FN;  // of one chunk
+    static constexpr int MFMAS = kTerms * T::FM * T::FN;  // of one chunk
 
     LA la[2];  // set j holds the steps s with s % 2 == j, loaded three ahead
     LB lb[2];
@@ -339,8 +316,7 @@ struct SplitEngine {
         b_store = LB::store_base(tid);
         a_read = ((lane >> 5) * SA::PLANE + wave / T::WAVES_N * T::WTM + (lane & 31)) * 16;
         b_read = ((lane >> 5) * SB::PLANE + wave % T::WAVES_N * T::WTN + (lane & 31)) * 16;
-        upper = 0xffff0000u;
-        asm("" : "+v"(upper));
+        upper = upper_half_mask();
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             la[q].init(lda, m0, m, tid);
@@ -376,9 +352,8 @@ struct SplitEngine {
     }
     // MFMA x of a chunk: column block x / (6 FM), term, row block.
     __device__ __forceinline__ void mfma(int x, const SplitFragments<T>& f) {
-        constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
-        const int j = x / (6 * T::FM), t = x / T::FM % 6, i = x % T::FM;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[kTerms[t][0]][i], f.b[kTerms[t][1]][j], acc[i][j], 0,
+        const int j = x / (kTerms * T::FM), t = x / T::FM % kTerms, i = x % T::FM;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[term_left(t)][i], f.b[term_right(t)][j], acc[i][j], 0,
                                                             0, 0);
     }
     // One K-step from the stage. NEXT: also splits set Q (the next step) into

@@ -127,12 +127,17 @@ struct CausalAttentionArgs {
     int64_t query_offset = 0;
     float scale = 1.f;
     // The context's workspace and arrival counters: the decode form (at most
-    // 4 queries per head, no probabilities) keeps per-chunk records there.
+    // 4 queries per head, no probabilities) and the key ranges of a launch with
+    // few query blocks keep their records there.
     float* workspace = nullptr;
     size_t workspace_bytes = 0;
     uint32_t* counters = nullptr;
     size_t counter_count = 0;
+    int cu_count = 256;
 };
+// The query-block form (attention_forward.hip), which launch_causal_attention
+// takes where the decode form does not apply.
+hipError_t launch_query_block_attention(const CausalAttentionArgs& args, hipStream_t stream);
 hipError_t launch_causal_attention(const CausalAttentionArgs& args, hipStream_t stream);
 // Head dims 32, 64, 128; 16-byte aligned pointers and strides; per-head
 // offsets within 31 bits.
