@@ -13,8 +13,8 @@
 // with D per query = sum over h of dO * O (equal to softmax_backward's
 // projection sum over keys of dP * P, since O = P V).
 //
-// Three launches, every sum taken in a fixed order (no atomics; reruns give
-// the same bits):
+// Up to four launches, every sum taken in a fixed order (no atomics; reruns
+// give the same bits):
 //  * rows: per query {m, 1 / l, D} into the workspace (12 bytes);
 //  * key blocks: a workgroup owns 128 keys of a head, a wave 32, with K and V
 //    of its keys in LDS (head dims 32, 64) or registers (128); Q, dO and the
@@ -24,6 +24,10 @@
 //    holds column l % 32, its key, so P and dS are already laid out as the B
 //    operands of dV^T += dO^T P and dK^T += Q^T dS (the forward's O^T +=
 //    V^T P^T, transposed roles);
+//    Head dims 32 and 64 with enough queries run them on the bf16 matrix cores
+//    from split operands (attention_key_grad_split.h); the fp32 kernels here
+//    keep the shorter sequences, head dim 128, and the blocks whose operands
+//    the split does not hold (a launch of their own);
 //  * dQ, one of two ways. Where the workspace holds them (head dims 32 and
 //    64), the key kernel also writes each stage's dS to LDS and multiplies it
 //    by the block's K, leaving per key block partial sums of dQ that a third
@@ -149,7 +153,18 @@ struct KeyGradArgs {
     float scale;
     float* partials;       // dQ partial sums (the LDS kernel's dQ form), else unused
     int64_t partial_rows;  // partial_rows() of the shape: rows per head
+    bool redo;             // after the split kernel: only the blocks it left to the fp32 instruction
 };
+
+constexpr int kLdsKeyWaves = 8;
+
+}  // namespace
+}  // namespace sn
+
+#include "attention_key_grad_split.h"
+
+namespace sn {
+namespace {
 
 // Element (row, h = 32 b + col) of a stage whose 16-byte chunks are
 // XOR-swizzled by row (slot (h / 4) ^ (row & SWIZZLE)), for the rows the
@@ -490,8 +505,6 @@ void attention_key_grad_kernel(KeyGradArgs a) {
 // order) and stores that part of the block's partial sums. The next stage's
 // loads are issued after the stage's first barrier, into the buffer the stage
 // before has finished with.
-constexpr int kLdsKeyWaves = 8;
-
 // The dS rows of a stage in LDS: row q holds the block's 128 keys, its 16-byte
 // chunk c stored at c ^ ds_swizzle(q). Bijective on the low four bits of c for
 // any 16 consecutive rows (the dQ step's reads, 16 rows at a time, cover all
@@ -504,6 +517,10 @@ template <int H, bool DQ = false>
 __global__ __launch_bounds__(64 * kLdsKeyWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attention_key_grad_lds_kernel(KeyGradArgs a) {
 #pragma clang fp contract(off)
+    if (a.redo) {
+        const float mark = a.k_grad[(blockIdx.x % a.heads * a.keys + blockIdx.x / a.heads * kKeyBlock) * H];
+        if (mark == mark) return;  // the split kernel's result stands
+    }
     using G = Geometry<H>;  // 64 queries per stage
     constexpr int W = kLdsKeyWaves;
     constexpr int LOADS = G::STAGE_SLOTS / (64 * W);  // stage loads per wave and operand
@@ -1098,6 +1115,24 @@ __global__ __launch_bounds__(256) void attention_dq_sum_kernel(DqSumArgs a) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// dK, dV (and the dQ partial sums): the split kernel, then the fp32 one for
+// the blocks it left. Few queries stay with the fp32 kernel alone: the second
+// launch costs 3 to 4 us, more than the split saves there.
+constexpr int64_t split_min_queries(int h) { return h == 32 ? 512 : 128; }
+
+template <int H, bool DQ>
+hipError_t launch_key_grad(KeyGradArgs a, int64_t key_blocks, hipStream_t stream) {
+    const dim3 grid(unsigned(a.heads * key_blocks)), block(64 * kLdsKeyWaves);
+    if (a.queries >= split_min_queries(H)) {
+        hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), grid, dim3(64 * kSplitWaves), 0, stream, a);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return err;
+        a.redo = true;
+    }
+    hipLaunchKernelGGL((attention_key_grad_lds_kernel<H, DQ>), grid, block, 0, stream, a);
+    return hipGetLastError();
+}
+
 template <int H>
 hipError_t launch_backward(const AttentionBackwardArgs& a, hipStream_t stream) {
     float* rows = a.workspace;
@@ -1108,7 +1143,7 @@ hipError_t launch_backward(const AttentionBackwardArgs& a, hipStream_t stream) {
     if (err != hipSuccess) return err;
 
     KeyGradArgs ka{a.q, a.k, a.v, a.d_out, rows, a.k_grad, a.v_grad, a.queries, a.keys, a.q_stride,
-                   a.kv_stride, a.query_offset, a.heads, a.scale, nullptr, 0};
+                   a.kv_stride, a.query_offset, a.heads, a.scale, nullptr, 0, false};
     const int64_t key_blocks = (a.keys + kKeyBlock - 1) / kKeyBlock;
     if constexpr (H <= 64) {
         // dQ from the key kernel's partial sums when the workspace holds them
@@ -1136,9 +1171,7 @@ hipError_t launch_backward(const AttentionBackwardArgs& a, hipStream_t stream) {
                 ra_.heads = n;
                 ra_.partials = partials;
                 ra_.partial_rows = prows;
-                hipLaunchKernelGGL((attention_key_grad_lds_kernel<H, true>), dim3(unsigned(n * key_blocks)),
-                                   dim3(64 * kLdsKeyWaves), 0, stream, ra_);
-                err = hipGetLastError();
+                err = launch_key_grad<H, true>(ra_, key_blocks, stream);
                 if (err != hipSuccess) return err;
                 DqSumArgs sa{partials, a.q_grad + h0 * a.queries * H, n, a.queries, a.keys, a.query_offset, prows,
                              a.scale};
@@ -1151,12 +1184,12 @@ hipError_t launch_backward(const AttentionBackwardArgs& a, hipStream_t stream) {
         }
     }
     if constexpr (H <= 64)
-        hipLaunchKernelGGL(attention_key_grad_lds_kernel<H>, dim3(unsigned(a.heads * key_blocks)),
-                           dim3(64 * kLdsKeyWaves), 0, stream, ka);
-    else
+        err = launch_key_grad<H, false>(ka, key_blocks, stream);
+    else {
         hipLaunchKernelGGL(attention_key_grad_kernel<H>, dim3(unsigned(a.heads * key_blocks)), dim3(64 * kWaves), 0,
                            stream, ka);
-    err = hipGetLastError();
+        err = hipGetLastError();
+    }
     if (err != hipSuccess) return err;
 
     QueryGradArgs qa{a.q, a.k, a.v, a.d_out, rows, a.q_grad, a.queries, a.keys, a.q_stride, a.kv_stride,
