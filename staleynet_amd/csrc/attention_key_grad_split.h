@@ -21,7 +21,10 @@
 //  * 79 KB of LDS at h = 64 (52 KB at 32): two workgroups a CU (three), so one's
 //    barriers, exponentials and splits run under the other's MFMAs. Eight waves
 //    with the rows stored in both orders (146 KB, one workgroup a CU, K and V in
-//    registers) left each wave's phases one after the other.
+//    registers) left each wave's phases one after the other: 2335 us for 192
+//    heads x 2048 x 64 against 1560-1670 (the fp32 kernel 2525; 165 TFLOP/s of
+//    its five products). LDS reads and MFMAs bound it about equally: 6900 and
+//    7700 cycles a CU for eight waves' blocks.
 //  * A block whose results are not finite, or hold a nonzero value under 2^-80
 //    (operands outside the split's range), leaves NaN as its first key's
 //    first dK; the fp32 kernel, launched after, computes the blocks that show
@@ -46,7 +49,8 @@ constexpr int kSplitQueries = 32;  // per stage
 // Stages between two additions of the dV and dK accumulators to memory: sums of
 // 1024 queries instead of one chain over all of them (error of the gradients of
 // 2048 queries against 64 bits: 7.4e-7 in one chain, the fp32 kernel's two
-// interleaved chains 6.8e-7).
+// interleaved chains 6.8e-7; flushed 5.6e-7, and every 512 queries 4.3e-7 for
+// 2 % more time).
 constexpr int kFlushStages = 32;
 
 // LDS of the kernel, in bytes. The planes' four spare slots put the octets a
