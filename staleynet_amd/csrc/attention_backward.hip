@@ -24,9 +24,9 @@
 //    holds column l % 32, its key, so P and dS are already laid out as the B
 //    operands of dV^T += dO^T P and dK^T += Q^T dS (the forward's O^T +=
 //    V^T P^T, transposed roles);
-//    Head dims 32 and 64 with enough queries run them on the bf16 matrix cores
+//    Head dims 32 and 64 run them on the bf16 matrix cores
 //    from split operands (attention_key_grad_split.h); the fp32 kernels here
-//    keep the shorter sequences, head dim 128, and the blocks whose operands
+//    keep head dim 128 and the blocks whose operands
 //    the split does not hold (a launch of their own);
 //  * dQ, one of two ways. Where the workspace holds them (head dims 32 and
 //    64), the key kernel also writes each stage's dS to LDS and multiplies it
@@ -1116,21 +1116,19 @@ __global__ __launch_bounds__(256) void attention_dq_sum_kernel(DqSumArgs a) {
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // dK, dV (and the dQ partial sums): the split kernel, then the fp32 one for
-// the blocks it left. Few queries stay with the fp32 kernel alone: the second
-// launch costs 3 to 4 us, more than the split saves there (training step of 8
-// heads, fp32 alone -> split: 64 x 64 44.0 -> 44.6 us, 128 x 64 62 -> 57.5, 256
-// x 32 64.0 -> 64.5, 520 x 32 105.3 -> 104.6).
-constexpr int64_t split_min_queries(int h) { return h == 32 ? 512 : 128; }
-
+// the blocks it left. Every length takes the
+// split: the forward's statistics come from split scores, and scores formed
+// another way here lose their agreement with them (8 heads x 64 x 64: dQ 3.6e-7
+// against 64 bits with the fp32 kernel after the split forward, 2.5e-7 with
+// this one; the second launch costs short sequences 2 us: 300 x 32 73 -> 75 us
+// a training step, 64 x 64 43.3 -> 44.7, 128 x 64 62 -> 58.6).
 template <int H, bool DQ>
 hipError_t launch_key_grad(KeyGradArgs a, int64_t key_blocks, hipStream_t stream) {
     const dim3 grid(unsigned(a.heads * key_blocks)), block(64 * kLdsKeyWaves);
-    if (a.queries >= split_min_queries(H)) {
-        hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), grid, dim3(64 * kSplitWaves), 0, stream, a);
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess) return err;
-        a.redo = true;
-    }
+    hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), grid, dim3(64 * kSplitWaves), 0, stream, a);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    a.redo = true;
     hipLaunchKernelGGL((attention_key_grad_lds_kernel<H, DQ>), grid, block, 0, stream, a);
     return hipGetLastError();
 }

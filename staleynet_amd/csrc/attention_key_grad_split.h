@@ -22,7 +22,7 @@
 //    barriers, exponentials and splits run under the other's MFMAs. Eight waves
 //    with the rows stored in both orders (146 KB, one workgroup a CU, K and V in
 //    registers) left each wave's phases one after the other: 2335 us for 192
-//    heads x 2048 x 64 against 1560-1670 (the fp32 kernel 2525; 165 TFLOP/s of
+//    heads x 2048 x 64 against 1540-1670 (the fp32 kernel 2525; 165 TFLOP/s of
 //    its five products). LDS reads and MFMAs bound it about equally: 6900 and
 //    7700 cycles a CU for eight waves' blocks.
 //  * A block whose results are not finite, or hold a nonzero value under 2^-80
@@ -46,12 +46,9 @@ __device__ __forceinline__ void hide(int& x) { asm volatile("" : "+v"(x)); }
 
 constexpr int kSplitWaves = 4;
 constexpr int kSplitQueries = 32;  // per stage
-// Stages between two additions of the dV and dK accumulators to memory: sums of
-// 1024 queries instead of one chain over all of them (error of the gradients of
-// 2048 queries against 64 bits: 7.4e-7 in one chain, the fp32 kernel's two
-// interleaved chains 6.8e-7; flushed 5.6e-7, and every 512 queries 4.3e-7 for
-// 2 % more time).
-constexpr int kFlushStages = 32;
+// Stages between two additions of the dV and dK accumulators to memory, so that
+// no chain of sums is longer than 2048 queries.
+constexpr int kFlushStages = 64;
 
 // LDS of the kernel, in bytes. The planes' four spare slots put the octets a
 // transposing load or an 8-byte write phase touches 64 bytes apart.
@@ -247,10 +244,16 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
                 const char* at = rows + column_read + p * S::ROW_PART + (4 * b * S::ROW_PLANE + 16 * c) * 16;
                 f[p] = transposed(at, at + 8 * 16);
             }
+            // The chunk's terms from zero, then one addition: the long sum is rounded once per 16 queries, not six
+            // times (2048 queries against 64 bits: 7.4e-7 with six, 3.3e-7 so; the fp32 kernel 6.8e-7).
+            f32x16 sum;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = 0.f;
 #pragma unroll
             for (int t = 0; t < kTerms; ++t)
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[term_left(t)], x.part[term_right(t)], acc[b], 0, 0,
-                                                                 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[term_left(t)], x.part[term_right(t)], sum, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[b][r] = acc[b][r] + sum[r];
         }
     };
     // This wave's block of the stage; dS split, register pairs (2 i, 2 i + 1), into ds.
