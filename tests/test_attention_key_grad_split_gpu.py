@@ -1,6 +1,6 @@
-"""The split key kernel of the attention backward (attention_key_grad_split.h) where it can go wrong: the shortest
-sequences it takes and those just under, ragged stages (32 queries) and key blocks (128), the flushes of its
-accumulators (every 512 queries), offsets; and operands outside the split's range, whose blocks the fp32 kernel
+"""The split key kernel of the attention backward (attention_key_grad_split.h) where it can go wrong: short
+sequences, ragged stages (32 queries) and key blocks (128), the flush of its accumulators (every 2048 queries),
+offsets; and operands outside the split's range, whose blocks the fp32 kernel
 computes again. Against the oracle's restatement of the reference's backward
 (crates/staleynet-model/src/layers/attention.rs:220-260) at the reference's fp32 tolerance."""
 import numpy as np
