@@ -107,10 +107,13 @@ extern "C" {
 /* Kernel selection, the role of the reference's MatmulKernel
  * (device.rs:38-67; public field Gpu::matmul_kernel, device.rs:144):
  *   SN_KERNEL_MFMA_F32  fp32 matrix-core GEMM (default; the role of Blocked);
- *                       tiled products split each fp32 operand exactly into
- *                       three bf16 parts and accumulate their products in
- *                       fp32 (nearer the 64-bit result than fp32 products
- *                       added one by one)
+ *                       tiled products of more than three terms split each
+ *                       fp32 operand exactly into three bf16 parts and
+ *                       accumulate six of their nine products in fp32 (those
+ *                       left out are under 2^-24 of a product). On dense
+ *                       operands that is nearer the 64-bit result than fp32
+ *                       products added one by one; a sum with one nonzero
+ *                       product is within 3 x 2^-24 of it
  *   SN_KERNEL_MFMA_BF16 inputs rounded to bf16 (nearest-even), fp32
  *                       accumulation (the role of TensorCore's TF32)
  *   SN_KERNEL_SIMPLE    one thread per output, k summed in order with

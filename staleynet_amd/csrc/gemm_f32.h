@@ -6,18 +6,24 @@
 // contract: any operand storage, strided batches, overwrite or accumulate,
 // zero padding of partial tiles, row-major output with row stride N.
 //
-// Arithmetic. An fp32 value is the exact sum of three bf16 values: hi, its
-// upper 16 bits; mid, the rest rounded to bf16; lo, what that leaves (at most
-// 8 bits, so exact). A product of two such sums has nine terms, each exact in
-// fp32 (8 x 8 bits); the six that reach 2^-24 of it are accumulated in fp32
-// by v_mfma_f32_32x32x16_bf16, smallest first, for every 16 k: lo hi, hi lo,
-// mid mid, mid hi, hi mid, hi hi. The three left out are below 2^-25 of the
-// product, of either sign. Per 16 k that is 6 roundings of an output where
-// v_mfma_f32_32x32x2_f32 rounds 16 times, so the result is nearer the 64-bit
-// one: relative 2-norm error 1.1e-7 / 2.4e-7 / 4.2e-7 / 8.6e-7 / 2.1e-6 at
-// K = 64 / 256 / 768 / 3072 / 16384 on N(0, 1) operands against 1.5e-7 /
-// 2.9e-7 / 5.0e-7 / 9.9e-7 / 2.3e-6 for the fp32 instruction, and 0.6 to 0.9
-// of it on positive and on widely spread operands.
+// Arithmetic. An fp32 value is the exact sum of three bf16 values: hi, the
+// value rounded to bf16; mid, the rest rounded to bf16; lo, what that leaves
+// (at most 7 bits, so exact). A product of two such sums has nine terms, each
+// exact in fp32 (8 x 8 bits); six are accumulated in fp32 by
+// v_mfma_f32_32x32x16_bf16, smallest first, for every 16 k: lo hi, hi lo, mid
+// mid, mid hi, hi mid, hi hi. The three left out are together under 2^-24 of
+// the product, of either sign. (With hi truncated they reached 2^-22, and
+// single products were off by 4.1e-8 rms and 4.3 x 2^-24 at worst.) Per 16 k
+// that is 6 roundings of an output where v_mfma_f32_32x32x2_f32 rounds 16
+// times. Relative 2-norm error on N(0, 1) operands at K = 4 / 64 / 768 / 3072 /
+// 16384: 3.2e-8 / 1.10e-7 / 2.41e-7 / 2.52e-7 / 3.6e-7 against 4.0e-8 /
+// 1.45e-7 / 2.89e-7 / 2.94e-7 / 3.8e-7 for the fp32 instruction, and 0.8 to 0.99
+// of it on positive and on widely spread operands (the larger K split over
+// workgroups as launched). Up to three products the fp32 instruction's few
+// roundings are the better ones (2.5e-8 for one), so it computes those
+// (kFewProducts). A row with a single nonzero entry among more keeps the
+// split's own error of one product: 3.5e-8 rms, 2.6 x 2^-24 at worst (0 where
+// one factor has 8 bits, a power of two or a small whole number).
 //  * Range. The split holds for every finite operand above 2^-109 in
 //    magnitude (below, lo's last bits pass the bf16 subnormals). An infinite
 //    or NaN operand makes its outputs NaN here, and outputs whose operands
@@ -417,6 +423,10 @@ struct SplitEngine {
     }
 };
 
+// Products per output (of a K slice) up to which the fp32 instruction's few
+// roundings err less than the split.
+constexpr int kFewProducts = 3;
+
 // Outputs under this magnitude (and not 0) are recomputed: an operand whose
 // last bits the split loses is under 2^-109, and one that large partner (over
 // 2^29) would have to lift such a product past the floor.
@@ -591,7 +601,7 @@ __device__ __forceinline__ void split_tile(const Args& args) {
         if (s + 1 < steps) e.template step<1, true>([&] { before(I1{}, k0 + T::BK); }, [&] {});
         e.template step<0, false>([&] {}, [&] {});
     }
-    if (needs_f32<T>(e.acc))
+    if (k_end - k_begin <= kFewProducts || needs_f32<T>(e.acc))
         recompute_f32<T, A_K, B_K>(args, a, b, m0, n0, k_begin, k_end, wave_m, wave_n, lane, e.acc);
 
     const bool partial = args.splits > 1;

@@ -22,10 +22,15 @@ __device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair_f32{lo, hi}, pair_bf16));
 }
 
-constexpr int kParts = 3;  // hi, mid, lo
+constexpr int kParts = 3;  // hi, mid, lo: each the rest so far rounded to bf16
 
-// The terms of a product of two split values that reach 2^-24 of it, smallest
-// first (parts of the left and of the right factor).
+// The six terms of a product of two split values that are kept, smallest first
+// (parts of the left and of the right factor). With hi within 2^-8 of the
+// value's power of two, mid is at most 2^-8 and lo 2^-17 of it, so the three
+// terms left out (mid lo, lo mid, lo lo) are together under 2^-24 of the
+// product. (Splitting fp32 into bf16 parts for the matrix cores: Henry, Tang
+// and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019.)
 constexpr int kTerms = 6;
 __host__ __device__ constexpr int term_left(int t) { return t == 0 ? 2 : t == 2 || t == 3 ? 1 : 0; }
 __host__ __device__ constexpr int term_right(int t) { return t == 1 ? 2 : t == 2 || t == 4 ? 1 : 0; }
@@ -38,23 +43,21 @@ __device__ __forceinline__ uint32_t upper_half_mask() {
     return mask;
 }
 
-// One third of the split of a pair of values: piece 0 takes hi (the upper 16
-// bits) and leaves the rests in x0 and x1, piece 1 takes mid (the rest
-// rounded), piece 2 lo (what that leaves: at most 8 bits, exact).
+// One third of the split of a pair of values: piece 0 takes hi (the value
+// rounded to nearest) and leaves the rests in x0 and x1, piece 1 takes mid (the
+// rest rounded), piece 2 lo (what that leaves: at most 7 bits, exact). A value
+// within 2^-9 of the largest float rounds to an infinite hi and leaves NaN.
 __device__ __forceinline__ void split_piece(int piece, float& x0, float& x1, uint32_t upper, uint32_t& hi,
                                             uint32_t& mid, uint32_t& lo) {
-    if (piece == 0) {
-        const uint32_t b0 = __builtin_bit_cast(uint32_t, x0), b1 = __builtin_bit_cast(uint32_t, x1);
-        hi = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-        x0 = x0 - __builtin_bit_cast(float, b0 & upper);
-        x1 = x1 - __builtin_bit_cast(float, b1 & upper);
-    } else if (piece == 1) {
-        mid = pack2_bf16(x0, x1);
-        x0 = x0 - __builtin_bit_cast(float, mid << 16);
-    } else {
+    if (piece == 2) {
         x1 = x1 - __builtin_bit_cast(float, mid & upper);
         lo = pack2_bf16(x0, x1);
+        return;
     }
+    uint32_t& part = piece == 0 ? hi : mid;
+    part = pack2_bf16(x0, x1);
+    x0 = x0 - __builtin_bit_cast(float, part << 16);
+    if (piece == 0) x1 = x1 - __builtin_bit_cast(float, part & upper);
 }
 
 __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t upper, uint32_t& hi, uint32_t& mid,

@@ -5,6 +5,8 @@ of its tiles, against the float64 product:
 - wide spreads of magnitude, within the bound of an fp32 sum in any order, (K + 8) 2^-24 sum |a| |b|;
 - operands near the smallest normal numbers (outputs the kernel recomputes with the fp32 instruction), the same
   bound plus K of the smallest subnormal;
+- sums of one to four products, where the split's own error shows: one product is rounded once, and up to four are
+  within the terms left out plus one rounding;
 - infinities and NaN: the same outputs are NaN or infinite (with the same sign) as in the float64 product, the
   others within the bound."""
 import numpy as np
@@ -35,7 +37,7 @@ def run(gpu, layout, m, n, k, a, b, tile):
     if layout[1] == "T":
         spec, right = spec.right_transposed(), b.T
     plan = gemm.plan(spec, cu_count=256)
-    assert (plan.tile_rows, plan.tile_cols) == tile, (plan.tile_rows, plan.tile_cols)
+    assert tile is None or (plan.tile_rows, plan.tile_cols) == tile, (plan.tile_rows, plan.tile_cols)
     print(f"{layout} {m}x{n}x{k} path {plan.path}", flush=True)
     lt = gpu.upload(Shape.vector(m * k), np.ascontiguousarray(left).ravel())
     rt = gpu.upload(Shape.vector(k * n), np.ascontiguousarray(right).ravel())
@@ -87,3 +89,23 @@ def test_infinities_nan_and_the_largest_values(gpu, layout, m, n, k, tile):
     a[1, :] = np.ldexp(a[1, :], -20)
     b[:, 1] = 0.0  # infinity times zero
     check(run(gpu, layout, m, n, k, a, b, tile), a, b, k)
+
+
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,n", [(128, 60), (260, 132), (2052, 4100)])  # every tile, by the alignment of k too
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_sums_of_few_products(gpu, layout, m, n, k):
+    # Values with the largest rests a split by truncation leaves among mantissas of every kind. Past K = 1: the terms
+    # left out are under 2^-24 of each product, the last addition rounds by 2^-24 of the sum, the five before it
+    # (2^-8 of it and less) are within 2^-6 of that.
+    rng = np.random.default_rng(m + k)
+    a = (rng.uniform(1, 2, (m, k)) * rng.choice([-1, 1], (m, k))).astype(np.float32)
+    b = rng.uniform(1, 2, (k, n)).astype(np.float32)
+    worst = np.array([0x3f80ff80], np.uint32).view(np.float32)[0]
+    a[::3], b[:, ::2] = worst, worst
+    got = run(gpu, layout, m, n, k, a, b, None)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    if k == 1:
+        assert np.array_equal(got, exact.astype(np.float32))
+    bound = (2 + 2.0 ** -6) * EPS * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.max(np.abs(got - exact) / bound) <= 1.0
