@@ -113,7 +113,11 @@ extern "C" {
  *                       left out are under 2^-24 of a product). On dense
  *                       operands that is nearer the 64-bit result than fp32
  *                       products added one by one; a sum with one nonzero
- *                       product is within 3 x 2^-24 of it
+ *                       product is within 3 x 2^-24 of it. Tiles with operands
+ *                       that three bf16 values do not hold (nonzero under
+ *                       2^-110, infinite, NaN or within 2^-9 of the largest
+ *                       float) are computed in fp32, at about a third of the
+ *                       speed
  *   SN_KERNEL_MFMA_BF16 inputs rounded to bf16 (nearest-even), fp32
  *                       accumulation (the role of TensorCore's TF32)
  *   SN_KERNEL_SIMPLE    one thread per output, k summed in order with

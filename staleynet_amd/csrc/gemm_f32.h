@@ -24,13 +24,20 @@
 // (kFewProducts). A row with a single nonzero entry among more keeps the
 // split's own error of one product: 3.5e-8 rms, 2.6 x 2^-24 at worst (0 where
 // one factor has 8 bits, a power of two or a small whole number).
-//  * Range. The split holds for every finite operand above 2^-109 in
-//    magnitude (below, lo's last bits pass the bf16 subnormals). An infinite
-//    or NaN operand makes its outputs NaN here, and outputs whose operands
-//    are all tiny lose precision. So a wave looks at its accumulators before
-//    it writes them (needs_f32), and one that holds a non-finite or a
-//    nonzero value under 2^-80 recomputes its part of the tile with the fp32
-//    instruction from the operands in memory (recompute_f32).
+//  * Range. The split holds zeros and every finite operand from 2^-110 on
+//    (split_bf16.h) up to 2^-9 under the largest float. The values of a step
+//    are looked at before they are split (note_set); a workgroup that has met
+//    a smaller one computes its tile again with the fp32 instruction from the
+//    operands in memory (recompute_f32), and so does a wave whose outputs are
+//    not finite (an infinite, NaN or largest operand, or an overflow). The
+//    operands decide, not the outputs: a tiny operand with a huge partner
+//    gives outputs of any size, and subnormal ones can leave 0. The look
+//    costs 1.7 % of a large product (32768 x 768 x 2304, a Linear step: 1860
+//    -> 1893 us), 3.5 % of the smallest tiled ones (it waits for a step's
+//    loads at once) and 3 % more where operands hold zeros (each value's
+//    range then); three instructions per pair as each is split, which zeros
+//    do not slow, cost 3 to 4 %. A tile computed again takes 3.5 times as
+//    long (4096 cubed with one such operand in each tile 865 -> 2995 us).
 //  * Six bf16 MFMAs do the work of eight fp32 ones (16 k of a 32 x 32 block)
 //    in 192 matrix-core cycles instead of 512. What bounds the kernel is
 //    power: on random operands six products' worth of MFMAs alone run at
@@ -169,6 +176,15 @@ struct SplitLoaderK {
             for (int e = 0; e < 4; ++e)
                 if (k0 + 4 * group(tid) + e > row0 + row(tid, v) + query_offset) reg[v][e] = 0.f;
     }
+    // f(x0, x1) of every pair of values held.
+    template <class F>
+    __device__ __forceinline__ void pairs(F&& f) const {
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+            f(reg[v][0], reg[v][1]);
+            f(reg[v][2], reg[v][3]);
+        }
+    }
     __device__ __forceinline__ static int store_base(int tid) {
         return (group(tid) / 2 * Stage::PLANE + tid / 8) * 16 + 8 * (group(tid) % 2);
     }
@@ -258,6 +274,14 @@ struct SplitLoaderR {
             for (int e = 0; e < N; ++e)
                 if (row0 + first_row(tid) + e > k0 + first_k(tid) + kk + query_offset) reg[kk][e] = 0.f;
     }
+    template <class F>
+    __device__ __forceinline__ void pairs(F&& f) const {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            f(reg[0][e], reg[1][e]);
+            f(reg[2][e], reg[3][e]);
+        }
+    }
     __device__ __forceinline__ static int store_base(int tid) {
         const int r = first_row(tid);
         return (tid / 64 * Stage::PLANE + (PAIRED ? r / 64 * 64 + r % 64 / 2 : r)) * 16 + 8 * (tid % 2);
@@ -312,8 +336,9 @@ struct SplitEngine {
     char* stage_b;
     int a_store, b_store, a_read, b_read;
     uint32_t upper;
+    uint32_t* mark;  // this wave's word in LDS: 1 once it has split a value the split does not hold
 
-    __device__ __forceinline__ void init(char* sa, char* sb, int tid, int64_t lda, int64_t ldb, int64_t m0, int64_t m,
+    __device__ __forceinline__ void init(char* sa, char* sb, uint32_t* marks, int tid, int64_t lda, int64_t ldb, int64_t m0, int64_t m,
                                          int64_t n0, int64_t n) {
         stage_a = sa;
         stage_b = sb;
@@ -323,6 +348,8 @@ struct SplitEngine {
         a_read = ((lane >> 5) * SA::PLANE + wave / T::WAVES_N * T::WTM + (lane & 31)) * 16;
         b_read = ((lane >> 5) * SB::PLANE + wave % T::WAVES_N * T::WTN + (lane & 31)) * 16;
         upper = upper_half_mask();
+        mark = marks + wave;
+        *mark = 0;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             la[q].init(lda, m0, m, tid);
@@ -337,9 +364,30 @@ struct SplitEngine {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     }
+    // Marks set Q's values for this wave if the split does not hold one: the
+    // smallest magnitude first (half an instruction a value), each value's
+    // range only where that is under the range (or 0).
+    template <int Q>
+    __device__ __forceinline__ void note_set() {
+        float m = 1.f;
+        auto smallest = [&](float x0, float x1) __attribute__((always_inline)) {
+            m = fminf(fminf(m, fabsf(x0)), fabsf(x1));
+            asm("" : "+v"(m));  // one running value, as in note_range
+        };
+        la[Q].pairs(smallest);
+        lb[Q].pairs(smallest);
+        if (__any(m < kSplitLeast)) {
+            uint32_t least = ~0u;
+            auto note = [&](float x0, float x1) __attribute__((always_inline)) { note_range(x0, x1, least); };
+            la[Q].pairs(note);
+            lb[Q].pairs(note);
+            if (least < kSplitLeastKey) *mark = 1;
+        }
+    }
     // Splits set Q into the stage (the first step, before any MFMA).
     template <int Q>
     __device__ __forceinline__ void stage_set() {
+        note_set<Q>();
 #pragma unroll
         for (int p = 0; p < LA::PIECES; ++p) la[Q].piece(p, upper, stage_a, a_store);
 #pragma unroll
@@ -395,23 +443,25 @@ struct SplitEngine {
         constexpr int FIRST = 2 * T::FM;  // MFMAs before the barrier
         constexpr int PIECES = LA::PIECES + LB::PIECES;
 #pragma unroll
-        for (int x = 0; x < MFMAS; ++x) {
-            if constexpr (NEXT) {
-                if (x == FIRST) {
-                    split_barrier();  // every wave holds both chunks' fragments
-                    before();
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+        for (int x = 0; x < FIRST; ++x) {
+            mfma(x, f1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (NEXT) {
+            split_barrier();  // every wave holds both chunks' fragments
+            before();
+            note_set<Q>();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int x = FIRST; x < MFMAS; ++x) {
             mfma(x, f1);
             if constexpr (NEXT) {
-                if (x >= FIRST) {
 #pragma unroll
-                    for (int p = (x - FIRST) * PIECES / (MFMAS - FIRST); p < (x - FIRST + 1) * PIECES / (MFMAS - FIRST);
-                         ++p) {
-                        if (p < LA::PIECES) la[Q].piece(p, upper, stage_a, a_store);
-                        else lb[Q].piece(p - LA::PIECES, upper, stage_b, b_store);
-                    }
+                for (int p = (x - FIRST) * PIECES / (MFMAS - FIRST); p < (x - FIRST + 1) * PIECES / (MFMAS - FIRST);
+                     ++p) {
+                    if (p < LA::PIECES) la[Q].piece(p, upper, stage_a, a_store);
+                    else lb[Q].piece(p - LA::PIECES, upper, stage_b, b_store);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -427,39 +477,27 @@ struct SplitEngine {
 // roundings err less than the split.
 constexpr int kFewProducts = 3;
 
-// Outputs under this magnitude (and not 0) are recomputed: an operand whose
-// last bits the split loses is under 2^-109, and one that large partner (over
-// 2^29) would have to lift such a product past the floor.
-constexpr float kSplitFloor = 0x1p-80f;
-
-// Whether a wave's accumulators hold a non-finite or a tiny nonzero value.
+// Whether a wave's accumulators hold a value that is not finite.
 template <class T>
-__device__ __forceinline__ bool needs_f32(const f32x16 (&acc)[T::FM][T::FN]) {
-    float poison = 0.f, least = 1.f;
+__device__ __forceinline__ bool not_finite(const f32x16 (&acc)[T::FM][T::FN]) {
+    float poison = 0.f;
 #pragma unroll
     for (int i = 0; i < T::FM; ++i)
 #pragma unroll
         for (int j = 0; j < T::FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float x = acc[i][j][r], y = acc[i][j][r + 1];
-                poison = __builtin_fmaf(x, 0.f, poison);  // NaN from the first non-finite value on
-                poison = __builtin_fmaf(y, 0.f, poison);
-                least = fminf(fminf(least, fabsf(x)), fabsf(y));
-            }
-    if (!__any(poison != 0.f || least < kSplitFloor)) return false;
-    // Exact zeros (rows and columns past the matrix, sparse operands) stay.
-    bool redo = false;
+            for (int r = 0; r < 16; ++r) poison = __builtin_fmaf(acc[i][j][r], 0.f, poison);  // NaN from then on
+    return __any(poison != 0.f);
+}
+
+// Whether a wave of the workgroup has split a value the split does not hold
+// (after the barrier that follows the last split).
+template <class T>
+__device__ __forceinline__ bool marked(const uint32_t (&marks)[T::THREADS / 64]) {
+    uint32_t any = 0;
 #pragma unroll
-    for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < T::FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float x = fabsf(acc[i][j][r]);
-                redo = redo || !(x < __builtin_inff()) || (x < kSplitFloor && x != 0.f);
-            }
-    return __any(redo);
+    for (int w = 0; w < T::THREADS / 64; ++w) any |= marks[w];
+    return __builtin_amdgcn_readfirstlane(any) != 0;
 }
 
 // A wave's blocks again, by v_mfma_f32_32x32x2_f32 on the operands as they
@@ -516,6 +554,7 @@ __device__ __forceinline__ void split_tile(const Args& args) {
     using LB = typename Engine::LB;
     __shared__ __attribute__((aligned(16))) char stage_a[Engine::SA::BYTES];
     __shared__ __attribute__((aligned(16))) char stage_b[Engine::SB::BYTES];
+    __shared__ __attribute__((aligned(16))) uint32_t marks[T::THREADS / 64];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -551,7 +590,7 @@ __device__ __forceinline__ void split_tile(const Args& args) {
     const float* b_origin = b + (B_K ? n0 * args.ldb : n0);
 
     Engine e;
-    e.init(stage_a, stage_b, tid, args.lda, args.ldb, m0, args.m, n0, args.n);
+    e.init(stage_a, stage_b, marks, tid, args.lda, args.ldb, m0, args.m, n0, args.n);
     e.clear();
     auto load = [&](auto set, int64_t k0) __attribute__((always_inline)) {
         constexpr int Q = decltype(set)::value;
@@ -601,7 +640,7 @@ __device__ __forceinline__ void split_tile(const Args& args) {
         if (s + 1 < steps) e.template step<1, true>([&] { before(I1{}, k0 + T::BK); }, [&] {});
         e.template step<0, false>([&] {}, [&] {});
     }
-    if (k_end - k_begin <= kFewProducts || needs_f32<T>(e.acc))
+    if (marked<T>(marks) || k_end - k_begin <= kFewProducts || not_finite<T>(e.acc))
         recompute_f32<T, A_K, B_K>(args, a, b, m0, n0, k_begin, k_end, wave_m, wave_n, lane, e.acc);
 
     const bool partial = args.splits > 1;

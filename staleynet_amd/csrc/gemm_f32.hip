@@ -30,6 +30,8 @@ void gemm_f32_persistent_kernel(Args args) {
     using Engine = SplitEngine<T, A_K, B_K, kLoadVector>;
     __shared__ __attribute__((aligned(16))) char stage_a[Engine::SA::BYTES];
     __shared__ __attribute__((aligned(16))) char stage_b[Engine::SB::BYTES];
+    // Of the item being computed and of the next, by turns.
+    __shared__ __attribute__((aligned(16))) uint32_t marks[2][T::THREADS / 64];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -53,7 +55,8 @@ void gemm_f32_persistent_kernel(Args args) {
 
     Engine e;
     // Whole tiles only: the loaders' offsets are the same for every item.
-    e.init(stage_a, stage_b, tid, args.lda, args.ldb, 0, T::BM, 0, T::BN);
+    marks[1][wave] = 0;
+    e.init(stage_a, stage_b, marks[0], tid, args.lda, args.ldb, 0, T::BM, 0, T::BN);
     // The next step to load: its item's tile origins, k and K end. Past the
     // workgroup's last item every load is out of range (k at the K end).
     int ld_w = w;
@@ -87,18 +90,24 @@ void gemm_f32_persistent_kernel(Args args) {
     e.template stage_set<0>();
     load_next(I0{});
     split_barrier();
-    for (;;) {
+    for (int turn = 0;; turn ^= 1) {
         const Item cur = item_of(w);
         const int64_t k_begin = k_begin_of(cur), k_end = k_end_of(cur);
         const int steps = int((k_end - k_begin + T::BK - 1) / T::BK);  // even (checked on the host)
         e.clear();
         for (int s = 0; s < steps; s += 2) {
-            e.template step<1, true>([] {}, [&] { load_next(I1{}); });
-            e.template step<0, true>([] {}, [&] { load_next(I0{}); });
+            e.template step<1, true>([] {},
+                                     [&] {
+                                         // Every wave is done with the item before: its words are the next one's.
+                                         if (s == 0) marks[turn ^ 1][wave] = 0;
+                                         load_next(I1{});
+                                     });
+            e.template step<0, true>([&] { e.mark = marks[s + 2 >= steps ? turn ^ 1 : turn] + wave; },
+                                     [&] { load_next(I0{}); });
         }
         const int64_t batch = args.batch_base + cur.batch_local;
         const int64_t m0 = int64_t(cur.tm) * T::BM, n0 = int64_t(cur.tn) * T::BN;
-        if (needs_f32<T>(e.acc))
+        if (marked<T>(marks[turn]) || not_finite<T>(e.acc))
             recompute_f32<T, A_K, B_K>(args, args.a + batch * args.stride_a, args.b + batch * args.stride_b, m0, n0,
                                        k_begin, k_end, wave_m, wave_n, lane, e.acc);
         const bool partial = args.splits > 1;

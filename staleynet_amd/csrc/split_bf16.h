@@ -43,6 +43,18 @@ __device__ __forceinline__ uint32_t upper_half_mask() {
     return mask;
 }
 
+// The split is exact for zeros and from 2^-110 on: there a value's last bit is
+// 2^-133 or more, bf16's smallest subnormal (the matrix cores keep subnormal
+// factors, products and sums). range_key orders values by magnitude with zeros
+// last, so that the least key of many tells whether the split holds them all.
+constexpr float kSplitLeast = 0x1p-110f;
+constexpr uint32_t kSplitLeastKey = 2 * (17u << 23) - 1;  // of kSplitLeast
+__device__ __forceinline__ uint32_t range_key(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 1; }
+__device__ __forceinline__ void note_range(float x0, float x1, uint32_t& least) {
+    least = min(min(least, range_key(x0)), range_key(x1));
+    asm("" : "+v"(least));  // one running value: keys gathered first would take registers
+}
+
 // One third of the split of a pair of values: piece 0 takes hi (the value
 // rounded to nearest) and leaves the rests in x0 and x1, piece 1 takes mid (the
 // rest rounded), piece 2 lo (what that leaves: at most 7 bits, exact). A value

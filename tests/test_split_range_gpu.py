@@ -3,8 +3,9 @@
 Every layout and tile (128 x 128, 128 x 64, 64 x 64, persistent; 16-byte and 4-byte-aligned loads), at the edges
 of its tiles, against the float64 product:
 - wide spreads of magnitude, within the bound of an fp32 sum in any order, (K + 8) 2^-24 sum |a| |b|;
-- operands near the smallest normal numbers (outputs the kernel recomputes with the fp32 instruction), the same
-  bound plus K of the smallest subnormal;
+- operands the split does not hold (nonzero under 2^-110; the kernel computes such tiles again with the fp32
+  instruction), of every size down to the subnormals, with ordinary and with huge partners, whatever the size of
+  the outputs: the same bound plus K of the smallest subnormal;
 - sums of one to four products, where the split's own error shows: one product is rounded once, and up to four are
   within the terms left out plus one rounding;
 - infinities and NaN: the same outputs are NaN or infinite (with the same sign) as in the float64 product, the
@@ -71,6 +72,26 @@ def test_spread_and_tiny_operands(gpu, layout, m, n, k, tile):
     # Rows of magnitude 2^-115 .. 2^-126, whose lowest bits no bf16 holds, and subnormal ones.
     tiny = np.ldexp(a, -110 - (np.arange(m) % 30)[:, None]).astype(np.float32)
     check(run(gpu, layout, m, n, k, tiny, b, tile), tiny, b, k)
+
+
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,n,k,tile", SHAPES, ids=IDS)
+def test_tiny_operands_with_huge_partners(gpu, layout, m, n, k, tile):
+    rng = np.random.default_rng(m * k + n)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    for down, up in ((-112, 30), (-120, 60), (-136, 118), (-140, 0)):
+        x, y = np.ldexp(a, down), np.ldexp(b, up)
+        check(run(gpu, layout, m, n, k, x, y, tile), x, y, k)
+        check(run(gpu, layout, m, n, k, np.ldexp(a, up), np.ldexp(b, down), tile), np.ldexp(a, up), np.ldexp(b, down), k)
+    # One tiny column, the only one of some rows, with a huge partner row; the last k and row of ragged tiles too.
+    for column, row in ((k // 2, 0), (k - 1, m - 1)):
+        x, y = a.copy(), b.copy()
+        x[:, column] = np.ldexp(a[:, column], -125)
+        y[column] = np.ldexp(b[column], 110)
+        for r in {row, m // 2}:
+            x[r, :column] = 0.0
+            x[r, column + 1:] = 0.0
+        check(run(gpu, layout, m, n, k, x, y, tile), x, y, k)
 
 
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
