@@ -35,9 +35,15 @@
 //    32-key block, then rescaled), so parity is to the fp32 tolerance.
 //  * Only the 32-key blocks on a wave's diagonal (or past the last key) test
 //    keys against each query's horizon; the others skip the mask.
-//  * A wave whose output or sum is not finite, or holds a nonzero value under
-//    2^-80 (operands outside the split's range), recomputes its queries with
-//    the fp32 instruction straight from memory.
+//  * Operands outside the split's range (split_bf16.h): each thread looks at the
+//    K and V it splits, and a wave at its Q. A wave with such a value among its
+//    operands, with an output or sum that is not finite or with no finite
+//    score recomputes its queries with the fp32 instruction straight from
+//    memory. The softmax's own e^(x - m) need no look: the exponential unit
+//    gives 0 under 2^-126 (as it did before the split), and the split is off by
+//    2^-134 at most on the ones between that and 2^-110, against sums of 1 or
+//    more. (The look costs 0.4 us of a prompt chunk's 20, and half a percent of
+//    a long sequence's training step.)
 //  * P (optional) takes a second pass over K with the final m and l: p =
 //    e^(s * scale - m) * (1 / l), 0 past the diagonal, so it matches the
 //    probabilities causal_softmax leaves to the fp32 tolerance.
@@ -144,6 +150,22 @@ struct KvLoader {
                 }
             }
     }
+    // f(x0, x1) of every pair of values held.
+    template <class F>
+    __device__ __forceinline__ void pairs(F&& f, bool with_v) const {
+#pragma unroll
+        for (int u = 0; u < KN; ++u) {
+            f(k[u][0], k[u][1]);
+            f(k[u][2], k[u][3]);
+        }
+        if (!with_v) return;
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                for (int e = 0; e < VN; e += 2) f(v[b][kk][e], v[b][kk][e + 1]);
+    }
     __device__ __forceinline__ void store(char* k_stage, char* v_stage, int tid, uint32_t upper, bool with_v) const {
         const int group = tid % G;
         char* kp = k_stage + (group / 2 * S::K_PLANE + tid / G) * 16 + 8 * (group % 2);
@@ -192,6 +214,8 @@ void causal_attention_kernel(AttentionArgs args) {
     constexpr int SUBS = kKeys / 32;
     __shared__ __attribute__((aligned(16))) char k_stage[kParts * S::K_PART];
     __shared__ __attribute__((aligned(16))) char v_stage[kParts * S::V_PART];
+    // Per wave: 1 once it has staged a value the split does not hold.
+    __shared__ __attribute__((aligned(16))) uint32_t marks[kWaves];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -233,13 +257,22 @@ void causal_attention_kernel(AttentionArgs args) {
             x[4 + s] = ok ? hi[s] : 0.f;
         }
     };
+    marks[wave] = 0;
+    float qv[CHUNKS][8];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) load_query(c, qv[c]);
+    KvLoader<H> kv;
+    kv.load(k_rsrc, v_rsrc, key_first, wg_keys, tid, true);
+    // Whether this lane's Q is not what the split holds.
+    const bool outside = out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+            for (int s = 0; s < 8; s += 2) f(qv[c][s], qv[c][s + 1]);
+    });
     SplitVector qs[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-        float x[8];
-        load_query(c, x);
-        qs[c] = split_vector(x, upper);
-    }
+    for (int c = 0; c < CHUNKS; ++c) qs[c] = split_vector(qv[c], upper);
 
     // S^T for 32 keys (rows 32 sub .. +31 of the stage) against this wave's queries.
     const int k_read = (half * S::K_PLANE + col) * 16;
@@ -343,10 +376,9 @@ void causal_attention_kernel(AttentionArgs args) {
     const int64_t wave_horizon = q_wave + args.query_offset;  // last key the wave's first query sees
     // A block is whole for the wave when its first query sees every key of it (wave-uniform).
     auto whole = [&](int64_t sub0) { return sub0 + 31 <= wave_horizon && sub0 + 32 <= wg_keys; };
-    KvLoader<H> kv;
-    kv.load(k_rsrc, v_rsrc, key_first, wg_keys, tid, true);
     for (int st = 0; st < stages_total; ++st) {
         const int64_t key0 = key_first + int64_t(st) * kKeys;
+        if (out_of_range([&](auto f) __attribute__((always_inline)) { kv.pairs(f, true); })) marks[wave] = 1;
         kv.store(k_stage, v_stage, tid, upper, true);
         kv.load(k_rsrc, v_rsrc, key0 + kKeys, wg_keys, tid, true);  // past the last key: zeros, no traffic
         lds_barrier();
@@ -381,25 +413,16 @@ void causal_attention_kernel(AttentionArgs args) {
         }
         return acc;
     };
-    bool redo = false;
-    {
-        float poison = __builtin_fmaf(l, 0.f, 0.f), least = 1.f;
+    float poison = l * 0.f;
 #pragma unroll
-        for (int b = 0; b < OBLOCKS; ++b)
+    for (int b = 0; b < OBLOCKS; ++b)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                poison = __builtin_fmaf(o[b][r], 0.f, poison);  // NaN from the first non-finite value on
-                least = fminf(least, fabsf(o[b][r]));
-            }
-        if (__any(poison != 0.f || least < 0x1p-80f)) {
-            bool bad = poison != 0.f;
-#pragma unroll
-            for (int b = 0; b < OBLOCKS; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) bad = bad || (o[b][r] != 0.f && fabsf(o[b][r]) < 0x1p-80f);
-            redo = __any(bad);
-        }
-    }
+        for (int r = 0; r < 16; ++r) poison = __builtin_fmaf(o[b][r], 0.f, poison);  // NaN from the first non-finite value on
+    // A query that sees a key of the range has a finite maximum, unless its scores overflowed.
+    const bool sees = q < args.queries && q + args.query_offset >= key_first;
+    const bool marked = (marks[0] | marks[1] | marks[2] | marks[3]) != 0;
+    static_assert(kWaves == 4, "the waves' marks");
+    const bool redo = __any(outside || marked || poison != 0.f || (sees && m == -INFINITY));
     if (redo) {
         clear();
         for (int64_t sub0 = key_first; sub0 < wave_keys; sub0 += 32) {

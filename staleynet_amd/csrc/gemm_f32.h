@@ -364,25 +364,14 @@ struct SplitEngine {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     }
-    // Marks set Q's values for this wave if the split does not hold one: the
-    // smallest magnitude first (half an instruction a value), each value's
-    // range only where that is under the range (or 0).
+    // Marks this wave if set Q holds a value that the split does not.
     template <int Q>
     __device__ __forceinline__ void note_set() {
-        float m = 1.f;
-        auto smallest = [&](float x0, float x1) __attribute__((always_inline)) {
-            m = fminf(fminf(m, fabsf(x0)), fabsf(x1));
-            asm("" : "+v"(m));  // one running value, as in note_range
-        };
-        la[Q].pairs(smallest);
-        lb[Q].pairs(smallest);
-        if (__any(m < kSplitLeast)) {
-            uint32_t least = ~0u;
-            auto note = [&](float x0, float x1) __attribute__((always_inline)) { note_range(x0, x1, least); };
-            la[Q].pairs(note);
-            lb[Q].pairs(note);
-            if (least < kSplitLeastKey) *mark = 1;
-        }
+        if (out_of_range([&](auto f) __attribute__((always_inline)) {
+                la[Q].pairs(f);
+                lb[Q].pairs(f);
+            }))
+            *mark = 1;
     }
     // Splits set Q into the stage (the first step, before any MFMA).
     template <int Q>

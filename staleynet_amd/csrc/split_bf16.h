@@ -55,6 +55,23 @@ __device__ __forceinline__ void note_range(float x0, float x1, uint32_t& least) 
     asm("" : "+v"(least));  // one running value: keys gathered first would take registers
 }
 
+// Whether this lane holds a value that the split does not; `pairs` calls its
+// argument with every pair of values. The smallest magnitude first (half an
+// instruction a value), each value's range only where a lane of the wave has
+// one under the range, or 0.
+template <class Pairs>
+__device__ __forceinline__ bool out_of_range(Pairs&& pairs) {
+    float m = 1.f;
+    pairs([&](float x0, float x1) __attribute__((always_inline)) {
+        m = fminf(fminf(m, fabsf(x0)), fabsf(x1));
+        asm("" : "+v"(m));  // one running value, as in note_range
+    });
+    if (!__any(m < kSplitLeast)) return false;
+    uint32_t least = ~0u;
+    pairs([&](float x0, float x1) __attribute__((always_inline)) { note_range(x0, x1, least); });
+    return least < kSplitLeastKey;
+}
+
 // One third of the split of a pair of values: piece 0 takes hi (the value
 // rounded to nearest) and leaves the rests in x0 and x1, piece 1 takes mid (the
 // rest rounded), piece 2 lo (what that leaves: at most 7 bits, exact). A value
