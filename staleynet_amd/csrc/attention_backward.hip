@@ -13,21 +13,18 @@
 // with D per query = sum over h of dO * O (equal to softmax_backward's
 // projection sum over keys of dP * P, since O = P V).
 //
-// Up to four launches, every sum taken in a fixed order (no atomics; reruns
-// give the same bits):
+// Three launches, every sum taken in a fixed order (no atomics; reruns give
+// the same bits):
 //  * rows: per query {m, 1 / l, D} into the workspace (12 bytes);
-//  * key blocks: a workgroup owns 128 keys of a head, a wave 32, with K and V
-//    of its keys in LDS (head dims 32, 64) or registers (128); Q, dO and the
-//    rows stream through LDS in 64-query stages, from the first query that
-//    sees the block to the last. A wave computes S = Q K^T and dP = dO V^T
-//    for 32 queries against its 32 keys: in the 32x32 accumulator lane l
-//    holds column l % 32, its key, so P and dS are already laid out as the B
-//    operands of dV^T += dO^T P and dK^T += Q^T dS (the forward's O^T +=
-//    V^T P^T, transposed roles);
-//    Head dims 32 and 64 run them on the bf16 matrix cores
-//    from split operands (attention_key_grad_split.h); the fp32 kernels here
-//    keep head dim 128 and the blocks whose operands
-//    the split does not hold (a launch of their own);
+//  * key blocks: a workgroup owns 128 keys of a head, a wave 32; Q, dO and the
+//    rows stream through LDS in stages, from the first query that sees the
+//    block to the last. A wave computes S = Q K^T and dP = dO V^T for 32
+//    queries against its 32 keys: in the 32x32 accumulator lane l holds column
+//    l % 32, its key, so P and dS are already laid out as the B operands of
+//    dV^T += dO^T P and dK^T += Q^T dS (the forward's O^T += V^T P^T,
+//    transposed roles). Head dims 32 and 64 run them on the bf16 matrix cores
+//    from split operands (attention_key_grad_split.h), head dim 128 with the
+//    fp32 instruction, K and V of the block in registers;
 //  * dQ, one of two ways. Where the workspace holds them (head dims 32 and
 //    64), the key kernel also writes each stage's dS to LDS and multiplies it
 //    by the block's K, leaving per key block partial sums of dQ that a third
@@ -151,12 +148,9 @@ struct KeyGradArgs {
     int64_t query_offset;
     int64_t heads;
     float scale;
-    float* partials;       // dQ partial sums (the LDS kernel's dQ form), else unused
+    float* partials;       // dQ partial sums (the split kernel's dQ form), else unused
     int64_t partial_rows;  // partial_rows() of the shape: rows per head
-    bool redo;             // after the split kernel: only the blocks it left to the fp32 instruction
 };
-
-constexpr int kLdsKeyWaves = 8;
 
 }  // namespace
 }  // namespace sn
@@ -199,28 +193,6 @@ struct ChunkReads {
         for (int i = 0; i < 2 * G::CHUNKS; ++i) launder(off[i]);
     }
     // 32 rows (32 sub .. of the stage) against the 32 columns held in `reg`.
-    // The same, with the 32 columns' values read from LDS rows laid out as a
-    // stage (`rows`: the first of the 32; row r's swizzle is r & SWIZZLE,
-    // which is col & SWIZZLE for row 32 i + col, so the offsets are shared).
-    __device__ __forceinline__ f32x16 product_lds(const f32x4* stage, int sub, const f32x4* rows) const {
-        const char* base = reinterpret_cast<const char*>(stage) + 32 * sub * G::SLOTS * 16;
-        const char* other = reinterpret_cast<const char*>(rows);
-        f32x16 acc;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-#pragma unroll
-        for (int c = 0; c < G::CHUNKS; ++c) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(base + off[2 * c]);
-            const f32x4 hi = *reinterpret_cast<const f32x4*>(base + off[2 * c + 1]);
-            const f32x4 ylo = *reinterpret_cast<const f32x4*>(other + off[2 * c]);
-            const f32x4 yhi = *reinterpret_cast<const f32x4*>(other + off[2 * c + 1]);
-            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            const float y[8] = {ylo[0], ylo[1], ylo[2], ylo[3], yhi[0], yhi[1], yhi[2], yhi[3]};
-#pragma unroll
-            for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
-        }
-        return acc;
-    }
     __device__ __forceinline__ f32x16 product(const f32x4* stage, int sub, const float (&reg)[G::CHUNKS][8]) const {
         const char* base = reinterpret_cast<const char*>(stage) + 32 * sub * G::SLOTS * 16;
         f32x16 acc;
@@ -485,384 +457,6 @@ void attention_key_grad_kernel(KeyGradArgs a) {
     }
 }
 
-// Key blocks with K and V in LDS, for head dims 32 and 64: eight waves, each
-// taking a key group (32 keys) against a query half of every stage (wave w:
-// half w / 4, stage rows 32 (w / 4) .. + 31). No wave holds K or V in registers, so
-// two share each SIMD; the K and V rows are read from LDS by the same
-// swizzled chunk reads as the stage rows. At the end the two halves' partial
-// dV^T and dK^T meet in LDS and are added in a fixed order (half 0, then
-// half 1): deterministic. (K, V and the stages of h = 128 exceed the LDS, so
-// that head dim keeps the register kernel above.)
-//
-// With DQ the kernel also computes dQ, as partial sums per key block that
-// attention_dq_sum_kernel adds up in block order, so that no query kernel has
-// to recompute S and dP (five products' MFMAs per pair instead of seven). Each
-// stage then ends in two more steps: the waves write their dS blocks to LDS,
-// as the stage's [64 queries][128 keys], over the stage's own Q and dO rows
-// (h = 64; h = 32 has LDS to spare for a buffer of its own); then wave w
-// multiplies queries 16 (w % 4) .. + 15 of it by h columns (w / 4) H / 2 ..
-// + H / 2 - 1 of the block's K (16 x 16 x 4 MFMAs over the 128 keys, in key
-// order) and stores that part of the block's partial sums. The next stage's
-// loads are issued after the stage's first barrier, into the buffer the stage
-// before has finished with.
-// The dS rows of a stage in LDS: row q holds the block's 128 keys, its 16-byte
-// chunk c stored at c ^ ds_swizzle(q). Bijective on the low four bits of c for
-// any 16 consecutive rows (the dQ step's reads, 16 rows at a time, cover all
-// banks), and rows q and q + 4 (the two lane halves of a write) differ in bit 3
-// (they fill opposite halves of the banks).
-__device__ __forceinline__ int ds_swizzle(int q) { return (q & 15) ^ ((q & 4) << 1); }
-constexpr int kDsRow = kKeyBlock;  // floats per dS row
-
-template <int H, bool DQ = false>
-__global__ __launch_bounds__(64 * kLdsKeyWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attention_key_grad_lds_kernel(KeyGradArgs a) {
-#pragma clang fp contract(off)
-    if (a.redo) {
-        const float mark = a.k_grad[(blockIdx.x % a.heads * a.keys + blockIdx.x / a.heads * kKeyBlock) * H];
-        if (mark == mark) return;  // the split kernel's result stands
-    }
-    using G = Geometry<H>;  // 64 queries per stage
-    constexpr int W = kLdsKeyWaves;
-    constexpr int LOADS = G::STAGE_SLOTS / (64 * W);  // stage loads per wave and operand
-    constexpr int KV_SLOTS = kKeyBlock * G::SLOTS;
-    constexpr int KV_LOADS = KV_SLOTS / (64 * W);
-    static_assert(H <= 64 && G::STAGE_SLOTS % (64 * W) == 0 && KV_SLOTS % (64 * W) == 0, "whole loads per wave");
-    // Partial sums handed over at the end: 2 x OBLOCKS accumulators per lane
-    // of the four half-1 waves, group g's in stage buffer g.
-    constexpr int HANDOFF_FLOATS = 2 * G::OBLOCKS * 16 * 64;
-    static_assert(HANDOFF_FLOATS <= G::STAGE_SLOTS * 4, "a group's hand-off fits in a stage buffer");
-    // A stage's dS: 64 rows of the block's keys, over the stage's Q and dO
-    // rows when those are large enough (h = 64), else in a buffer of its own.
-    constexpr int DS_FLOATS = kKeys * kDsRow;
-    constexpr bool DS_OVER_STAGE = 2 * G::STAGE_SLOTS * 4 >= DS_FLOATS;
-    constexpr int DS_OWN = DQ && !DS_OVER_STAGE ? DS_FLOATS / 4 : 1;
-    // Each stage's Q and dO rows are one LDS object, apart from the other
-    // stage's: the compiler tracks the direct-to-LDS loads in flight per
-    // object, so the reads of one stage do not wait for the loads into the
-    // other (with one array for both stages it made every stage's first
-    // read wait for the next stage's loads).
-    __shared__ f32x4 kv_lds[2][KV_SLOTS];
-    __shared__ f32x4 stage0[2][G::STAGE_SLOTS], stage1[2][G::STAGE_SLOTS];  // [Q, dO]
-    __shared__ f32x4 r_stage0[W][64], r_stage1[W][64];
-    __shared__ f32x4 ds_own[DS_OWN];
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    auto q_of = [&](auto stage) __attribute__((always_inline)) -> f32x4* {
-        if constexpr (decltype(stage)::value == 0) return stage0[0];
-        else return stage1[0];
-    };
-    auto d_of = [&](auto stage) __attribute__((always_inline)) -> f32x4* {
-        if constexpr (decltype(stage)::value == 0) return stage0[1];
-        else return stage1[1];
-    };
-    auto r_of = [&](auto stage) __attribute__((always_inline)) -> f32x4* {
-        if constexpr (decltype(stage)::value == 0) return r_stage0[0];
-        else return r_stage1[0];
-    };
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Key group and query half. Waves w and w + 4 share a SIMD: pairing group
-    // g of half 0 with group 3 - g of half 1 spreads the blocks of the two
-    // stages on the diagonal, where only groups up to the queries' reach
-    // work, over the SIMDs (with group g in both halves, the first stage's
-    // blocks fell on SIMDs 0 and 1 only).
-    const int group = wave < 4 ? wave : 7 - wave;
-    const int qh = wave / 4;
-    const int col = lane & 31;
-    const int half = lane >> 5;
-
-    const int64_t block = blockIdx.x;
-    const int64_t head = block % a.heads;
-    const int64_t k_first = (block / a.heads) * kKeyBlock;
-    const int64_t k_wave = k_first + 32 * group;
-    const int64_t key = k_wave + col;
-    const bool key_ok = key < a.keys;
-    const int64_t q_seen = max(int64_t(0), k_first - a.query_offset);
-    const int64_t q_begin = q_seen / kKeys * kKeys;
-    const int stages_total = q_begin < a.queries ? int((a.queries - q_begin + kKeys - 1) / kKeys) : 0;
-
-    const float* q_head = a.q + head * a.q_stride;
-    const float* d_head = a.d_out + head * a.q_stride;
-    const int64_t plane = plane_of(a.queries);
-    const float* r_head = a.rows + head * 3 * plane;
-
-    // K and V of the block's 128 keys into LDS, swizzled as the stages (rows
-    // past the last key read zeros).
-    {
-        const __amdgpu_buffer_rsrc_t k_rsrc = buffer_of(a.k + head * a.kv_stride + k_first * H);
-        const __amdgpu_buffer_rsrc_t v_rsrc = buffer_of(a.v + head * a.kv_stride + k_first * H);
-        const int32_t rows_left = int32_t(min(a.keys - k_first, int64_t(kKeyBlock)));
-#pragma unroll
-        for (int u = 0; u < KV_LOADS; ++u) {
-            const int e = 64 * (wave * KV_LOADS + u) + lane;
-            const int row = e / G::SLOTS;
-            const int32_t off = row < rows_left ? (row * H + 4 * ((e % G::SLOTS) ^ (row & G::SWIZZLE))) * 4 : kOutOfRange;
-            dma16(k_rsrc, kv_lds[0] + 64 * (wave * KV_LOADS + u), off);
-            dma16(v_rsrc, kv_lds[1] + 64 * (wave * KV_LOADS + u), off);
-        }
-    }
-    int32_t stage_row[LOADS], stage_off[LOADS];
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-        const int e = 64 * (wave * LOADS + u) + lane;
-        const int row = e / G::SLOTS;
-        stage_row[u] = row;
-        stage_off[u] = (row * H + 4 * ((e % G::SLOTS) ^ (row & G::SWIZZLE))) * 4;
-    }
-    const int32_t record_off = int32_t(((lane / 16) * plane + 4 * (lane % 16)) * 4);
-
-    auto issue = [&](auto stage, int64_t q0) __attribute__((always_inline)) {
-        f32x4* qs = q_of(stage);
-        f32x4* ds = d_of(stage);
-        const __amdgpu_buffer_rsrc_t q_rsrc = buffer_of(q_head + q0 * H);
-        const __amdgpu_buffer_rsrc_t d_rsrc = buffer_of(d_head + q0 * H);
-        const int32_t rows_left = int32_t(min(a.queries - q0, int64_t(kKeys)));  // wave-uniform
-#pragma unroll
-        for (int u = 0; u < LOADS; ++u) {
-            const int32_t off = stage_row[u] < rows_left ? stage_off[u] : kOutOfRange;
-            dma16(q_rsrc, qs + 64 * (wave * LOADS + u), off);
-            dma16(d_rsrc, ds + 64 * (wave * LOADS + u), off);
-        }
-        const __amdgpu_buffer_rsrc_t r_rsrc = buffer_of(r_head + q0);
-        dma16(r_rsrc, r_of(stage) + 64 * wave, lane < 48 && 4 * (lane % 16) < rows_left ? record_off : kOutOfRange);
-    };
-    ColumnReads<H> columns(col, half);
-    ChunkReads<H> chunks(col, half);
-    f32x16 dv[G::OBLOCKS], dk[G::OBLOCKS];
-#pragma unroll
-    for (int b = 0; b < G::OBLOCKS; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            dv[b][r] = 0.f;
-            dk[b][r] = 0.f;
-        }
-
-    // This wave's block of a stage: queries sub0 .. + 31 (rows 32 qh ..)
-    // against its 32 keys, as the register kernel's block_grad; dS of row
-    // 8 g + 4 half + j of the block into ds_out[4 g + j].
-    auto block_grad = [&](auto stage, auto masked, int64_t sub0, float (&ds_out)[16]) __attribute__((always_inline)) {
-        constexpr bool MASKED = decltype(masked)::value;
-        const f32x4* qs = q_of(stage);
-        const f32x4* ds = d_of(stage);
-        int record = 64 * wave + half;
-        launder(record);
-        const f32x4* rs = r_of(stage) + record;
-        int kv_row = 32 * group * G::SLOTS;
-        launder(kv_row);
-        chunks.launder_all();
-        columns.launder_all();
-        const f32x16 s = chunks.product_lds(qs, qh, kv_lds[0] + kv_row);
-        __builtin_amdgcn_sched_barrier(0);
-        const f32x16 dp = chunks.product_lds(ds, qh, kv_lds[1] + kv_row);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            __builtin_amdgcn_sched_barrier(0);
-            const int slot = 8 * qh + 2 * g;
-            const f32x4 m4 = rs[slot], il4 = rs[16 + slot], d4 = rs[32 + slot];
-            float p[4], gr[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float shifted = s[4 * g + j] * a.scale - m4[j];
-                const float pr = exp_of(shifted) * il4[j];
-                const float difference = dp[4 * g + j] - d4[j];
-                const float grad = pr * difference;
-                if (MASKED) {
-                    // Both terms are selected, not scaled by a zero p: a record
-                    // slot past the last query may hold any bits, Inf and NaN included.
-                    const int64_t query = sub0 + 8 * g + 4 * half + j;
-                    const bool visible = key_ok && query < a.queries && key <= query + a.query_offset;
-                    p[j] = visible ? pr : 0.f;
-                    gr[j] = visible ? grad : 0.f;
-                } else {
-                    p[j] = pr;
-                    gr[j] = grad;
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < G::OBLOCKS; ++b)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    dv[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(columns.read(ds, qh, g, j, b), p[j], dv[b], 0, 0, 0);
-                    dk[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(columns.read(qs, qh, g, j, b), gr[j], dk[b], 0, 0, 0);
-                }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) ds_out[4 * g + j] = gr[j];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    using Masked = std::true_type;
-    using Whole = std::false_type;
-    // The wave's block of the stage; dS stays 0 for a skipped block.
-    auto compute = [&](auto stage, int64_t q0, float (&ds_out)[16]) __attribute__((always_inline)) {
-        const int64_t sub0 = q0 + 32 * qh;
-        // Wave-uniform: skipped when none of the block's queries sees the wave's first key.
-        if (sub0 < a.queries && sub0 + 31 + a.query_offset >= k_wave && k_wave < a.keys) {
-            if (sub0 + a.query_offset >= k_wave + 31 && sub0 + 32 <= a.queries && k_wave + 32 <= a.keys)
-                block_grad(stage, Whole{}, sub0, ds_out);
-            else
-                block_grad(stage, Masked{}, sub0, ds_out);
-        }
-    };
-    if constexpr (DQ) {
-        // The dQ step's share of wave w: stage rows 16 (w % 4) + (lane % 16)
-        // (B operand: dS[q][keys]) against h columns (w / 4) H / 2 + 16 t +
-        // (lane % 16) of K (A operand), t < H / 32; MFMA 4 u + e pairs the
-        // keys 16 u + 4 (lane / 16) + e. The 16 x 16 result in lane l:
-        // h = 4 (l / 16) + r, query l % 16, four consecutive h per lane.
-        constexpr int HT = H / 32;
-        const int h_base = (wave / 4) * (H / 2);
-        // Partial sums of this block: rows from its first stage's first query.
-        int64_t rows_before = 0;
-        for (int64_t b = 0; b < block / a.heads; ++b) rows_before += block_queries(b, a.queries, a.query_offset);
-        const __amdgpu_buffer_rsrc_t p_rsrc =
-            buffer_of(a.partials + (head * a.partial_rows + rows_before) * H);
-        constexpr int STORES = HT;  // partial-sum stores per wave per stage
-        auto dq_step = [&](auto stage, int64_t q0, const float (&ds_in)[16]) __attribute__((always_inline)) {
-            float* dsm = DS_OVER_STAGE ? reinterpret_cast<float*>(q_of(stage)) : reinterpret_cast<float*>(ds_own);
-            if constexpr (DS_OVER_STAGE) lds_barrier();  // every wave is done with the stage's Q and dO
-            // dS row 32 qh + 8 g + 4 half + j, key 32 group + col.
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int q = 32 * qh + 8 * g + 4 * half + j, kl = 32 * group + col;
-                    dsm[q * kDsRow + 4 * ((kl / 4) ^ ds_swizzle(q)) + (kl & 3)] = ds_in[4 * g + j];
-                }
-            lds_barrier();  // the stage's dS is whole
-            // Byte offsets of the A reads (K row 4 lg + e of each 16-key step,
-            // column h_base + 16 t + lq) and of the B reads (chunk 4 (u % 4) +
-            // lg of dS row dq_row); u / 4 and the steps add immediates. Formed
-            // here, from a laundered lane, rather than held through the stage.
-            int l = lane;
-            launder(l);
-            const int lq = l % 16, lg = l / 16;
-            const int dq_row = 16 * (wave % 4) + lq;  // stage row
-            int k_off[4][HT], d_off[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                for (int t = 0; t < HT; ++t) {
-                    const int row = 4 * lg + e, h = h_base + 16 * t + lq;
-                    k_off[e][t] = (row * H + 4 * ((h / 4) ^ (row & G::SWIZZLE)) + (h & 3)) * 4;
-                }
-                d_off[e] = (dq_row * kDsRow + 4 * ((4 * e + lg) ^ ds_swizzle(dq_row))) * 4;
-            }
-            f32x4 acc[HT];
-#pragma unroll
-            for (int t = 0; t < HT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const char* kb = reinterpret_cast<const char*>(kv_lds[0]);
-            const char* db = reinterpret_cast<const char*>(dsm);
-#pragma unroll
-            for (int u = 0; u < kDsRow / 16; ++u) {
-                const f32x4 d4 = *reinterpret_cast<const f32x4*>(db + d_off[u % 4] + (u / 4) * 256);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int t = 0; t < HT; ++t) {
-                        const float kv = *reinterpret_cast<const float*>(kb + k_off[e][t] + u * 16 * H * 4);
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, d4[e], acc[t], 0, 0, 0);
-                    }
-            }
-            // Rows past the last query are dropped (out-of-range offsets).
-            const int64_t q = q0 + dq_row;
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-            for (int t = 0; t < HT; ++t) {
-                const int32_t off = q < a.queries ? int32_t(((q - q_begin) * H + h_base + 16 * t + 4 * lg) * 4)
-                                                  : kOutOfRange;
-                // The row offset rides in the vector offset, soffset 0: with a
-                // scalar soffset the compiler may let the next VALU overwrite
-                // the data registers before this 4-dword store has read them.
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[t]), p_rsrc, off, 0, 0);
-            }
-        };
-        auto stage_dq = [&](auto stage, int64_t q0) __attribute__((always_inline)) {
-            float dsv[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dsv[i] = 0.f;
-            compute(stage, q0, dsv);
-            dq_step(stage, q0, dsv);
-        };
-        // Each stage starts once every wave is done with the stage before,
-        // whose buffer then takes the next stage's loads (past the last query
-        // they read zeros); it ends waiting for those loads, which leaves this
-        // wave's partial-sum stores in flight. The waits and loads are
-        // unconditional, so the compiler's count of the loads in flight stays
-        // exact and it adds no waits of its own.
-        issue(I0{}, q_begin);
-        wait_loads<0>();  // K, V and the first stage
-        for (int st = 0; st < stages_total; st += 2) {
-            const int64_t q0 = q_begin + int64_t(st) * kKeys;
-            lds_barrier();
-            issue(I1{}, q0 + kKeys);
-            stage_dq(I0{}, q0);
-            wait_loads<STORES>();
-            if (st + 1 >= stages_total) break;
-            lds_barrier();
-            issue(I0{}, q0 + 2 * kKeys);
-            stage_dq(I1{}, q0 + kKeys);
-            wait_loads<STORES>();
-        }
-    } else {
-        // K and V go first, so the first wait (all but one stage's loads)
-        // covers them too.
-        constexpr int kStageLoads = 2 * LOADS + 1;
-        float unused[16];
-        issue(I0{}, q_begin);
-        issue(I1{}, q_begin + kKeys);
-        for (int st = 0; st < stages_total; st += 2) {
-            const int64_t q0 = q_begin + int64_t(st) * kKeys;
-            wait_loads<kStageLoads>();
-            lds_barrier();
-            compute(I0{}, q0, unused);
-            lds_barrier();
-            issue(I0{}, q0 + 2 * kKeys);
-            wait_loads<kStageLoads>();
-            lds_barrier();
-            if (st + 1 < stages_total) compute(I1{}, q0 + kKeys, unused);
-            lds_barrier();
-            issue(I1{}, q0 + 3 * kKeys);
-        }
-    }
-    wait_loads<0>();
-    lds_barrier();  // every wave is done with the stages (and K, V)
-
-    // Half 1 hands its partial sums to half 0 through the stages' space
-    // (lane-consecutive, conflict-free); half 0 adds them and writes.
-    float* handoff = reinterpret_cast<float*>(group < 2 ? stage0[group] : stage1[group - 2]) + lane;
-    if (qh == 1) {
-#pragma unroll
-        for (int b = 0; b < G::OBLOCKS; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                handoff[((2 * b) * 16 + r) * 64] = dv[b][r];
-                handoff[((2 * b + 1) * 16 + r) * 64] = dk[b][r];
-            }
-    }
-    lds_barrier();
-    if (qh == 0 && key_ok) {
-        float* vrow = a.v_grad + (head * a.keys + key) * H;
-        float* krow = a.k_grad + (head * a.keys + key) * H;
-#pragma unroll
-        for (int b = 0; b < G::OBLOCKS; ++b)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                f32x4 vo, ko;
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int r = 4 * g + s;
-                    vo[s] = dv[b][r] + handoff[((2 * b) * 16 + r) * 64];
-                    const float sum = dk[b][r] + handoff[((2 * b + 1) * 16 + r) * 64];
-                    ko[s] = a.scale * sum;
-                }
-                *reinterpret_cast<f32x4*>(vrow + 32 * b + 4 * half + 8 * g) = vo;
-                *reinterpret_cast<f32x4*>(krow + 32 * b + 4 * half + 8 * g) = ko;
-            }
-    }
-}
-
 struct QueryGradArgs {
     const float* q;
     const float* k;
@@ -1115,21 +709,15 @@ __global__ __launch_bounds__(256) void attention_dq_sum_kernel(DqSumArgs a) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// dK, dV (and the dQ partial sums): the split kernel, then the fp32 one for
-// the blocks it left. Every length takes the
-// split: the forward's statistics come from split scores, and scores formed
+// dK, dV (and the dQ partial sums) of head dims 32 and 64. Every length takes
+// the split: the forward's statistics come from split scores, and scores formed
 // another way here lose their agreement with them (8 heads x 64 x 64: dQ 3.6e-7
-// against 64 bits with the fp32 kernel after the split forward, 2.5e-7 with
-// this one; the second launch costs short sequences 2 us: 300 x 32 73 -> 75 us
-// a training step, 64 x 64 43.3 -> 44.7, 128 x 64 62 -> 58.6).
+// against 64 bits with an fp32 kernel after the split forward, 2.5e-7 with this
+// one).
 template <int H, bool DQ>
-hipError_t launch_key_grad(KeyGradArgs a, int64_t key_blocks, hipStream_t stream) {
-    const dim3 grid(unsigned(a.heads * key_blocks)), block(64 * kLdsKeyWaves);
-    hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), grid, dim3(64 * kSplitWaves), 0, stream, a);
-    const hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    a.redo = true;
-    hipLaunchKernelGGL((attention_key_grad_lds_kernel<H, DQ>), grid, block, 0, stream, a);
+hipError_t launch_key_grad(const KeyGradArgs& a, int64_t key_blocks, hipStream_t stream) {
+    hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), dim3(unsigned(a.heads * key_blocks)),
+                       dim3(64 * kSplitWaves), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -1143,7 +731,7 @@ hipError_t launch_backward(const AttentionBackwardArgs& a, hipStream_t stream) {
     if (err != hipSuccess) return err;
 
     KeyGradArgs ka{a.q, a.k, a.v, a.d_out, rows, a.k_grad, a.v_grad, a.queries, a.keys, a.q_stride,
-                   a.kv_stride, a.query_offset, a.heads, a.scale, nullptr, 0, false};
+                   a.kv_stride, a.query_offset, a.heads, a.scale, nullptr, 0};
     const int64_t key_blocks = (a.keys + kKeyBlock - 1) / kKeyBlock;
     if constexpr (H <= 64) {
         // dQ from the key kernel's partial sums when the workspace holds them

@@ -25,10 +25,15 @@
 //    heads x 2048 x 64 against 1540-1670 (the fp32 kernel 2525; 165 TFLOP/s of
 //    its five products). LDS reads and MFMAs bound it about equally: 6900 and
 //    7700 cycles a CU for eight waves' blocks.
-//  * A block whose results are not finite, or hold a nonzero value under 2^-80
-//    (operands outside the split's range), leaves NaN as its first key's
-//    first dK; the fp32 kernel, launched after, computes the blocks that show
-//    NaN there again and leaves at once on the others.
+//  * Range (split_bf16.h): threads look at the Q, K, V and dO they split. P and
+//    dS are formed 2^64 times too large (the factor rides in the rows' 1 / l,
+//    and the sums are divided by it, exactly), so that every normal fp32 P or
+//    dS is one the split holds. A block with an operand outside the range, or
+//    with a sum that is not finite, is computed again by the same workgroup
+//    with the fp32 instruction from memory. (A backward whose every block is:
+//    192 heads x 1024 x 64 557 -> 1870 us. Peaked scores and gradients of a mean
+//    loss stay at 575. A launch of their own for such blocks cost every backward
+//    2 to 9 us.)
 #pragma once
 
 #include "attention_common.h"
@@ -50,6 +55,9 @@ constexpr int kSplitQueries = 32;  // per stage
 // no chain of sums is longer than 2048 queries.
 constexpr int kFlushStages = 64;
 
+// P and dS are formed this many times too large; 2^64 x 2^-64 = 1.
+constexpr float kGradScale = 0x1p64f, kGradUnscale = 0x1p-64f;
+
 // LDS of the kernel, in bytes. The planes' four spare slots put the octets a
 // transposing load or an 8-byte write phase touches 64 bytes apart.
 template <int H>
@@ -62,6 +70,8 @@ struct KeyGradStage {
     static constexpr int BYTES = 2 * ROWS > kParts * DS_PART ? 2 * ROWS : kParts * DS_PART;
     static constexpr int K_PLANE = kKeyBlock + 4;        // slots per octet of h (slot = key)
     static constexpr int K_PART = H / 8 * K_PLANE * 16;
+    static constexpr int DS_ROW = kSplitQueries + 1;     // floats per key of the recomputed dS
+    static_assert(kKeyBlock * DS_ROW * 4 <= BYTES, "the recomputed dS fits the stage");
 };
 
 // Four rows x 16 columns of 16-bit values per 16 lanes, transposed: lane 4 i +
@@ -96,7 +106,8 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
     __shared__ __attribute__((aligned(16))) char stage[S::BYTES];
     __shared__ __attribute__((aligned(16))) char k_lds[kParts * S::K_PART];
     __shared__ __attribute__((aligned(16))) float records[3 * kSplitQueries];
-    __shared__ int bad_waves[kSplitWaves];
+    // Per wave: 1 once its part of the block has to be computed again.
+    __shared__ __attribute__((aligned(16))) uint32_t marks[kSplitWaves];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -104,6 +115,7 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
     const int col = lane & 31;
     const int half = lane >> 5;
     const uint32_t upper = upper_half_mask();
+    marks[wave] = 0;
 
     const int64_t block = blockIdx.x;
     const int64_t head = block % a.heads;
@@ -119,39 +131,45 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
     const float* r_head = a.rows + head * 3 * plane;
     const __amdgpu_buffer_rsrc_t k_rsrc = buffer_of(a.k + head * a.kv_stride + k_first * H);
 
-    // A thread's four vectors of a stage: threads 0 .. 2 H - 1 take Q's, the
-    // next 2 H dO's (h = 32 leaves half the threads none); G consecutive
-    // threads read a row.
-    const int operand = wave / (H / 32);  // 0 Q, 1 dO, 2 and 3 none
+    // A thread's vectors of a stage: the first half of the threads take Q's rows,
+    // the other dO's; G consecutive threads read a row.
+    constexpr int VECTORS = H / 16;
+    constexpr int ROWS_APART = 32 * kSplitWaves / G;
+    const int operand = wave / 2;
     const int hg = tid % G;
-    const int row0 = tid % (2 * H) / G;   // rows row0 + 8 r
+    const int row0 = tid % (32 * kSplitWaves) / G;
     const float* o_head = (operand == 0 ? a.q : a.d_out) + head * a.q_stride;
-    const bool loads = operand < 2;
-    split_f32x4 next[4];
+    split_f32x4 next[VECTORS];
     float next_record = 0.f;
     auto load = [&](int64_t q0) __attribute__((always_inline)) {
         // Rows past the last query read zeros.
         const int left = int(min(max(a.queries - q0, int64_t(0)), int64_t(kSplitQueries)));
-        if (loads) {
-            const __amdgpu_buffer_rsrc_t rsrc = buffer_of(o_head + q0 * H);
+        const __amdgpu_buffer_rsrc_t rsrc = buffer_of(o_head + q0 * H);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int32_t off = row0 + 8 * r < left ? ((row0 + 8 * r) * H + 4 * hg) * 4 : kOutOfRange;
-                next[r] = __builtin_bit_cast(split_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
-            }
+        for (int r = 0; r < VECTORS; ++r) {
+            const int row = row0 + ROWS_APART * r;
+            const int32_t off = row < left ? (row * H + 4 * hg) * 4 : kOutOfRange;
+            next[r] = __builtin_bit_cast(split_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
         }
         if (tid < 3 * kSplitQueries) {
             const int q = tid % kSplitQueries;
             next_record = q < left ? r_head[(tid / kSplitQueries) * plane + q0 + q] : 0.f;
         }
     };
-    const int row_store = (loads ? operand : 0) * S::ROWS + (hg / 2 * S::ROW_PLANE + row0) * 16 + 8 * (hg % 2);
+    const int row_store = operand * S::ROWS + (hg / 2 * S::ROW_PLANE + row0) * 16 + 8 * (hg % 2);
     auto store = [&]() __attribute__((always_inline)) {
-        if (loads) {
+        if (out_of_range([&](auto f) __attribute__((always_inline)) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) put_split(stage + row_store + 8 * r * 16, S::ROW_PART, next[r], upper);
-        }
-        if (tid < 3 * kSplitQueries) records[tid] = next_record;
+                for (int r = 0; r < VECTORS; ++r) {
+                    f(next[r][0], next[r][1]);
+                    f(next[r][2], next[r][3]);
+                }
+            }))
+            marks[wave] = 1;
+#pragma unroll
+        for (int r = 0; r < VECTORS; ++r) put_split(stage + row_store + ROWS_APART * r * 16, S::ROW_PART, next[r], upper);
+        if (tid < 3 * kSplitQueries)
+            records[tid] = tid / kSplitQueries == 1 ? next_record * kGradScale : next_record;  // 1 / l scaled
     };
 
     load(q_begin);
@@ -165,6 +183,14 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
             const int32_t off = e / G < rows_left ? 16 * e : kOutOfRange;
             x[u] = __builtin_bit_cast(split_f32x4, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, off, 0, 0));
         }
+        if (out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < KN; ++u) {
+                    f(x[u][0], x[u][1]);
+                    f(x[u][2], x[u][3]);
+                }
+            }))
+            marks[wave] = 1;
 #pragma unroll
         for (int u = 0; u < KN; ++u)
             put_split(k_lds + (hg / 2 * S::K_PLANE + tid / G + u * 64 * kSplitWaves / G) * 16 + 8 * (hg % 2), S::K_PART,
@@ -173,27 +199,40 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     // V of this lane's key: chunk c holds h 16 c + 8 half + (0..7).
     SplitVector vs[CHUNKS];
+    {
+        float x[CHUNKS][8];
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-        const float* from = a.v + head * a.kv_stride + (key_ok ? key : 0) * H + 8 * half + 16 * c;
-        const split_f32x4 lo = *reinterpret_cast<const split_f32x4*>(from);
-        const split_f32x4 hi = *reinterpret_cast<const split_f32x4*>(from + 4);
-        float x[8];
+        for (int c = 0; c < CHUNKS; ++c) {
+            const float* from = a.v + head * a.kv_stride + (key_ok ? key : 0) * H + 8 * half + 16 * c;
+            const split_f32x4 lo = *reinterpret_cast<const split_f32x4*>(from);
+            const split_f32x4 hi = *reinterpret_cast<const split_f32x4*>(from + 4);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            x[s] = key_ok ? lo[s] : 0.f;
-            x[4 + s] = key_ok ? hi[s] : 0.f;
+            for (int s = 0; s < 4; ++s) {
+                x[c][s] = key_ok ? lo[s] : 0.f;
+                x[c][4 + s] = key_ok ? hi[s] : 0.f;
+            }
         }
-        vs[c] = split_vector(x, upper);
+        if (out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+                for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+                    for (int s = 0; s < 8; s += 2) f(x[c][s], x[c][s + 1]);
+            }))
+            marks[wave] = 1;
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) vs[c] = split_vector(x[c], upper);
     }
     f32x16 dv[OBLOCKS], dk[OBLOCKS];
+    auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < OBLOCKS; ++b)
+        for (int b = 0; b < OBLOCKS; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            dv[b][r] = 0.f;
-            dk[b][r] = 0.f;
-        }
+            for (int r = 0; r < 16; ++r) {
+                dv[b][r] = 0.f;
+                dk[b][r] = 0.f;
+            }
+    };
+    clear();
 
     // The stage's 32 queries (octets of h at `rows`) against this wave's keys,
     // whose chunk c right(c, part) gives. Each chunk's fragments are read under
@@ -282,7 +321,7 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
                     const float pr = exp_of(shifted) * il4[j];
                     const float difference = dp[8 * c + 4 * g + j] - d4[j];
                     p[4 * g + j] = at + j >= first ? pr : 0.f;
-                    gr[4 * g + j] = p[4 * g + j] * difference;  // NaN if dP is not finite: computed again in fp32
+                    gr[4 * g + j] = p[4 * g + j] * difference;  // NaN if dP is not finite: computed again
                 }
             }
             add_columns(stage + S::ROWS, c, split_vector(p, upper), dv);
@@ -309,10 +348,18 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
     // Word (keys col & ~1, + 1) of query row 4 half + (lane & 1) + ...
     const int ds_store = ((4 * wave + col / 8) * S::DS_PLANE + 4 * half + (lane & 1)) * 16 + col % 8 / 2 * 4;
     const uint32_t pick = lane & 1 ? 0x03020706u : 0x05040100u;
-    float poison = 0.f, least = 1.f;
+    float poison = 0.f;
     auto look = [&](float x) __attribute__((always_inline)) {
         poison = __builtin_fmaf(x, 0.f, poison);  // NaN from the first non-finite value on
-        least = fminf(least, x == 0.f ? 1.f : fabsf(x));
+    };
+    // dQ's 16 x 16 result: lane l's four h of query dq_row. Rows past the last query are dropped (out-of-range
+    // offsets).
+    auto store_partial = [&](int64_t q0, int dq_row, int lg, int t, split_f32x4 sum) __attribute__((always_inline)) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const int64_t q = q0 + dq_row;
+        const int32_t off =
+            q < a.queries ? int32_t(((q - q_begin) * H + h_base + 16 * t + 4 * lg) * 4) : kOutOfRange;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum), p_rsrc, off, 0, 0);
     };
     auto dq_step = [&](int64_t q0) __attribute__((always_inline)) {
         int l = lane;
@@ -349,22 +396,21 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
                 acc[x % HT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     f[x % 2][term_left(i)], d[x / HT % 2][term_right(i)], acc[x % HT], 0, 0, 0);
         }
-        // Rows past the last query are dropped (out-of-range offsets).
-        const int64_t q = q0 + dq_row;
-        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
         for (int t = 0; t < HT; ++t) {
-            const int32_t off =
-                q < a.queries ? int32_t(((q - q_begin) * H + h_base + 16 * t + 4 * lg) * 4) : kOutOfRange;
+            split_f32x4 sum;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) look(acc[t][r]);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[t]), p_rsrc, off, 0, 0);
+            for (int r = 0; r < 4; ++r) {
+                look(acc[t][r]);
+                sum[r] = acc[t][r] * kGradUnscale;
+            }
+            store_partial(q0, dq_row, lg, t, sum);
         }
     };
 
-    // dV = (dV^T)^T and dK = (dK^T)^T: lane l holds h rows 32 b + 4 half + 8 g + (0..3) of its key. Adds to
-    // what an earlier flush left (`add`); the last one scales dK, which `again` marks.
-    auto flush = [&](bool add, bool last, bool again) __attribute__((always_inline)) {
+    // dV = (dV^T)^T and dK = (dK^T)^T: lane l holds h rows 32 b + 4 half + 8 g + (0..3) of its key, times
+    // 1 / `unscale`. Adds to what an earlier flush left (`add`); the last one scales dK.
+    auto flush = [&](bool add, bool last, float unscale) __attribute__((always_inline)) {
         if (!key_ok) return;
         float* vrow = a.v_grad + (head * a.keys + key) * H + 4 * half;
         float* krow = a.k_grad + (head * a.keys + key) * H + 4 * half;
@@ -378,8 +424,8 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
                 split_f32x4 vo, ko;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    vo[s] = dv[b][4 * g + s];
-                    ko[s] = dk[b][4 * g + s];
+                    vo[s] = dv[b][4 * g + s] * unscale;
+                    ko[s] = dk[b][4 * g + s] * unscale;
                 }
                 if (add) {
                     const split_f32x4 v0 = *vp, k0 = *kp;
@@ -391,7 +437,6 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
                 }
 #pragma unroll
                 for (int s = 0; s < 4; ++s) ko[s] = scale * ko[s];
-                if (b == 0 && g == 0 && again) ko[0] = __builtin_nanf("");
                 *vp = vo;
                 *kp = ko;
             }
@@ -410,14 +455,8 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
         const int64_t q0 = q_begin + int64_t(st) * kSplitQueries;
         if (st > 0 && st % kFlushStages == 0) {
             look_all();
-            flush(st > kFlushStages, false, false);
-#pragma unroll
-            for (int b = 0; b < OBLOCKS; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    dv[b][r] = 0.f;
-                    dk[b][r] = 0.f;
-                }
+            flush(st > kFlushStages, false, kGradUnscale);
+            clear();
         }
         store();
         load(q0 + kSplitQueries);  // past the last query: zeros, no traffic
@@ -448,13 +487,81 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
         lds_barrier();  // and read
     }
     look_all();
-    const bool bad = __any(poison != 0.f || least < 0x1p-80f);
-    if (lane == 0) bad_waves[wave] = bad;
+    if (__any(poison != 0.f)) marks[wave] = 1;
     lds_barrier();
-    int any = 0;
+    static_assert(kSplitWaves == 4, "the waves' marks");
+    if (__builtin_amdgcn_readfirstlane(marks[0] | marks[1] | marks[2] | marks[3]) == 0) {
+        flush(stages_total > kFlushStages, true, kGradUnscale);
+        return;
+    }
+
+    // The block again with the fp32 instruction, operands from memory: S and dP a 32 x 32 block per wave as above, P
+    // and dS as they are, dS through LDS for dQ. Rare, and written for few registers.
+    clear();
+#pragma unroll 1
+    for (int64_t q0 = q_begin; q0 < a.queries; q0 += kSplitQueries) {
+        f32x16 s, dp;
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w) any |= bad_waves[w];
-    flush(stages_total > kFlushStages, true, any != 0 && tid == 0);  // thread 0: the block's first key, h from 0
+        for (int r = 0; r < 16; ++r) {
+            s[r] = 0.f;
+            dp[r] = 0.f;
+        }
+        const float* q_head = a.q + head * a.q_stride;
+        const float* d_head = a.d_out + head * a.q_stride;
+        const bool row_ok = q0 + col < a.queries;
+        const int64_t row = (row_ok ? q0 + col : 0) * H + 8 * half;
+        const int64_t kv_row = head * a.kv_stride + (key_ok ? key : 0) * H + 8 * half;
+#pragma unroll 1
+        for (int c = 0; c < CHUNKS; ++c) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float qv = q_head[row + 16 * c + i], dv_ = d_head[row + 16 * c + i];
+                const float kv = a.k[kv_row + 16 * c + i], vv = a.v[kv_row + 16 * c + i];
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(row_ok ? qv : 0.f, key_ok ? kv : 0.f, s, 0, 0, 0);
+                dp = __builtin_amdgcn_mfma_f32_32x32x2f32(row_ok ? dv_ : 0.f, key_ok ? vv : 0.f, dp, 0, 0, 0);
+            }
+        }
+        float* ds_lds = reinterpret_cast<float*>(stage) + (32 * wave + col) * S::DS_ROW;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int at = 8 * (r / 4) + 4 * half + r % 4;
+            const int64_t q = q0 + at;
+            const bool visible = key_ok && q < a.queries && key <= q + a.query_offset;
+            const float* record = r_head + (q < a.queries ? q : 0);
+            const float shifted = s[r] * a.scale - record[0];
+            const float p = exp_of(shifted) * record[plane];
+            const float g = p * (dp[r] - record[2 * plane]);
+            const float pr = visible ? p : 0.f, gr = visible ? g : 0.f;
+            ds_lds[at] = gr;
+            const float* qrow = q_head + (q < a.queries ? q : 0) * H + col;
+            const float* drow = d_head + (q < a.queries ? q : 0) * H + col;
+#pragma unroll
+            for (int b = 0; b < OBLOCKS; ++b) {
+                dv[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(q < a.queries ? drow[32 * b] : 0.f, pr, dv[b], 0, 0, 0);
+                dk[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(q < a.queries ? qrow[32 * b] : 0.f, gr, dk[b], 0, 0, 0);
+            }
+        }
+        if constexpr (DQ) {
+            lds_barrier();  // the stage's dS is whole
+            const int lq = lane % 16, lg = lane / 16;
+            const int dq_row = 16 * (wave % 2) + lq;
+#pragma unroll
+            for (int t = 0; t < HT; ++t) {
+                split_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+                for (int u = 0; u < kKeyBlock; u += 4) {
+                    const bool ok = k_first + u + lg < a.keys;
+                    const float kv = a.k[head * a.kv_stride + (ok ? k_first + u + lg : 0) * H + h_base + 16 * t + lq];
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        ok ? kv : 0.f, reinterpret_cast<const float*>(stage)[(u + lg) * S::DS_ROW + dq_row], acc, 0, 0,
+                        0);
+                }
+                store_partial(q0, dq_row, lg, t, acc);
+            }
+            lds_barrier();  // and read
+        }
+    }
+    flush(false, true, 1.f);
 }
 
 }  // namespace

@@ -1,7 +1,7 @@
 """The split key kernel of the attention backward (attention_key_grad_split.h) where it can go wrong: short
 sequences, ragged stages (32 queries) and key blocks (128), the flush of its accumulators (every 2048 queries),
-offsets; and operands outside the split's range, whose blocks the fp32 kernel
-computes again. Against the oracle's restatement of the reference's backward
+offsets; and operands outside the split's range or gradients too large for its scaled sums, whose blocks it
+computes again with the fp32 instruction. Against the oracle's restatement of the reference's backward
 (crates/staleynet-model/src/layers/attention.rs:220-260) at the reference's fp32 tolerance."""
 import numpy as np
 import pytest
@@ -30,13 +30,25 @@ def test_edges_match_the_reference_calls(gpu, heads, queries, keys, h, offset):
         assert oracle.relative_error(expected, got[name]) < TOLERANCE, name
 
 
-def backward(gpu, q, k, v, d_out, heads, queries, keys, h, scale):
+def exact(q, k, v, d_out, heads, queries, keys, h, scale, offset):
+    q, k, v, d_out = (x.reshape(heads, -1, h).astype(np.float64) for x in (q, k, v, d_out))
+    scale = np.float64(np.float32(scale))
+    visible = np.arange(keys)[None, :] <= np.arange(queries)[:, None] + offset
+    s = np.where(visible, scale * (q @ k.transpose(0, 2, 1)), -np.inf)
+    p = np.exp(s - s.max(axis=2, keepdims=True))
+    p /= p.sum(axis=2, keepdims=True)
+    ds = p * (d_out @ v.transpose(0, 2, 1) - np.sum(d_out * (p @ v), axis=2, keepdims=True))
+    return scale * (ds @ k), scale * (ds.transpose(0, 2, 1) @ q), p.transpose(0, 2, 1) @ d_out
+
+
+def backward(gpu, q, k, v, d_out, heads, queries, keys, h, scale, offset=0):
+    print(f"heads={heads} queries={queries} keys={keys} h={h} offset={offset}", flush=True)
     Q, K, V, dO = (gpu.upload(Shape.vector(x.size), x) for x in (q, k, v, d_out))
     O, dQ = (gpu.zeros(Shape.vector(heads * queries * h)) for _ in range(2))
     dK, dV = (gpu.zeros(Shape.vector(heads * keys * h)) for _ in range(2))
     stats = gpu.zeros(Shape.vector(2 * heads * queries))
-    gpu.causal_attention_with_stats(Q, K, V, O, stats, heads, queries, keys, h, scale, 0)
-    gpu.causal_attention_backward(Q, K, V, O, dO, stats, dQ, dK, dV, heads, queries, keys, h, scale, 0)
+    gpu.causal_attention_with_stats(Q, K, V, O, stats, heads, queries, keys, h, scale, offset)
+    gpu.causal_attention_backward(Q, K, V, O, dO, stats, dQ, dK, dV, heads, queries, keys, h, scale, offset)
     got = [gpu.download(t) for t in (dQ, dK, dV)]
     for t in (Q, K, V, dO, O, stats, dQ, dK, dV):
         t.free()
@@ -81,3 +93,38 @@ def test_a_bad_query_reaches_what_it_sees_and_no_more(gpu, h, value):
                        ("dv", ev[0], dv[0])):
         assert np.all(np.isfinite(g)), name
         assert oracle.relative_error(e.ravel(), g.ravel()) < TOLERANCE, name
+
+
+@pytest.mark.parametrize("h", [32, 64])
+@pytest.mark.parametrize("heads,queries,keys,offset", [(2, 300, 300, 0), (1, 131, 257, 126), (1, 2100, 130, 0)])
+@pytest.mark.parametrize("powers", [dict(q=-122, k=122), dict(q=122, k=-122), dict(v=-124), dict(d=-124),
+                                    dict(v=-60, d=-62), dict(d=70), dict(v=65, d=-10)],
+                         ids=lambda p: " ".join(f"{n} 2^{e}" for n, e in p.items()))
+def test_operands_outside_the_range(gpu, h, heads, queries, keys, offset, powers):
+    # Scores stay of ordinary size; the gradients are scaled by powers of two, so their norms are taken in float64.
+    scale = h ** -0.5
+    rng = np.random.default_rng(h + queries)
+    sizes = dict(q=queries, k=keys, v=keys, d=queries)
+    q, k, v, d = (np.ldexp(rng.standard_normal(heads * n * h).astype(np.float32), powers.get(name, 0))
+                  for name, n in sizes.items())
+    expected = exact(q, k, v, d, heads, queries, keys, h, scale, offset)
+    got = backward(gpu, q, k, v, d, heads, queries, keys, h, scale, offset)
+    for name, e, g in zip(("dq", "dk", "dv"), expected, got):
+        assert np.all(np.isfinite(g)), name
+        assert np.linalg.norm(g.astype(np.float64) - e.ravel()) / np.linalg.norm(e) < TOLERANCE, name
+
+
+@pytest.mark.parametrize("h", [32, 64])
+def test_peaked_scores_and_small_gradients(gpu, h):
+    # Scores with gaps of 60 and more and dO of 2^-80: P dO of keys that hardly any query weighs is near the smallest
+    # normal fp32. Each key's dV (sums without cancellation) relative to its own size, down to 2^-100; the weights'
+    # own error is |s - m| 2^-24 and a few roundings, under 1e-5 for the gaps that matter there (100 2^-24).
+    heads, queries, scale = 2, 400, h ** -0.5
+    rng = np.random.default_rng(h + 9)
+    q, k, v, d = (rng.standard_normal((heads, queries, h)).astype(np.float32) for _ in range(4))
+    q, k, d = 3 * q, 3 * k, np.ldexp(np.abs(d), -80)
+    *_, expected = exact(q, k, v, d, heads, queries, queries, h, scale, 0)
+    *_, got = backward(gpu, *(x.ravel() for x in (q, k, v, d)), heads, queries, queries, h, scale)
+    rows = np.linalg.norm(expected, axis=2)
+    error = np.linalg.norm(got.reshape(expected.shape).astype(np.float64) - expected, axis=2)
+    assert np.min(rows) < 2.0 ** -80 and np.max((error / rows)[rows > 2.0 ** -100]) < TOLERANCE
