@@ -25,6 +25,9 @@
 //    transposed roles). Head dims 32 and 64 run them on the bf16 matrix cores
 //    from split operands (attention_key_grad_split.h), head dim 128 with the
 //    fp32 instruction, K and V of the block in registers;
+//    S has the forward's bits in every kernel (block_scores: split operands;
+//    192 heads x 1024 x 64 against 64 bits with fp32 scores instead: dQ of the
+//    query kernel 4.3e-7, now 3.8e-7; head dim 128 dQ 5.2e-7, now 4.4e-7);
 //  * dQ, one of two ways. Where the workspace holds them (head dims 32 and
 //    64), the key kernel also writes each stage's dS to LDS and multiplies it
 //    by the block's K, leaving per key block partial sums of dQ that a third
@@ -44,6 +47,7 @@
 
 #include "attention_common.h"
 #include "gemm_internal.h"
+#include "split_bf16.h"
 
 namespace sn {
 namespace {
@@ -192,6 +196,27 @@ struct ChunkReads {
 #pragma unroll
         for (int i = 0; i < 2 * G::CHUNKS; ++i) launder(off[i]);
     }
+    // The scores of 32 stage rows and the 32 columns held in `reg` (reg_outside: a lane's are not what the split holds).
+    template <bool KEYS_LEFT>
+    __device__ __forceinline__ f32x16 scores(const f32x4* stage, int sub, const float (&reg)[G::CHUNKS][8],
+                                             bool reg_outside, uint32_t upper) const {
+        const char* base = reinterpret_cast<const char*>(stage) + 32 * sub * G::SLOTS * 16;
+        return block_scores<H, KEYS_LEFT, G::CHUNKS>(
+            [&](int c, float (&x)[8]) __attribute__((always_inline)) {
+                const f32x4 lo = *reinterpret_cast<const f32x4*>(base + off[2 * c]);
+                const f32x4 hi = *reinterpret_cast<const f32x4*>(base + off[2 * c + 1]);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    x[s] = lo[s];
+                    x[4 + s] = hi[s];
+                }
+            },
+            [&](int c, float (&y)[8]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int s = 0; s < 8; ++s) y[s] = reg[c][s];
+            },
+            reg_outside, upper);
+    }
     // 32 rows (32 sub .. of the stage) against the 32 columns held in `reg`.
     __device__ __forceinline__ f32x16 product(const f32x4* stage, int sub, const float (&reg)[G::CHUNKS][8]) const {
         const char* base = reinterpret_cast<const char*>(stage) + 32 * sub * G::SLOTS * 16;
@@ -318,6 +343,15 @@ void attention_key_grad_kernel(KeyGradArgs a) {
         }
     }
 
+    // Whether this lane's K is not what the split holds.
+    const bool outside = out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < G::CHUNKS; ++c)
+#pragma unroll
+            for (int s = 0; s < 8; s += 2) f(kreg[c][s], kreg[c][s + 1]);
+    });
+    const uint32_t upper = upper_half_mask();
+
     // Q and dO rows of a stage, swizzled as the forward stages K; the rows'
     // records into this wave's copy.
     auto issue = [&](auto stage, int64_t q0) __attribute__((always_inline)) {
@@ -364,7 +398,7 @@ void attention_key_grad_kernel(KeyGradArgs a) {
         const f32x4* rs = r_of(stage) + record;
         chunks.launder_all();
         columns.launder_all();
-        const f32x16 s = chunks.product(qs, sub, kreg);
+        const f32x16 s = chunks.template scores<false>(qs, sub, kreg, outside, upper);
         __builtin_amdgcn_sched_barrier(0);
         const f32x16 dp = chunks.product(ds, sub, vreg);
 #pragma unroll
@@ -547,6 +581,15 @@ void attention_query_grad_kernel(QueryGradArgs a) {
         }
     }
 
+    // Whether this lane's Q is not what the split holds.
+    const bool outside = out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < G::CHUNKS; ++c)
+#pragma unroll
+            for (int s = 0; s < 8; s += 2) f(qreg[c][s], qreg[c][s + 1]);
+    });
+    const uint32_t upper = upper_half_mask();
+
     // K and V rows of a stage, both swizzled (K is read by chunks for S^T and
     // element by element for K^T).
     auto issue = [&](auto stage, int64_t key0) __attribute__((always_inline)) {
@@ -580,7 +623,7 @@ void attention_query_grad_kernel(QueryGradArgs a) {
         const f32x4* ks = k_of(stage);
         chunks.launder_all();
         columns.launder_all();
-        const f32x16 s = chunks.product(ks, sub, qreg);
+        const f32x16 s = chunks.template scores<true>(ks, sub, qreg, outside, upper);
         __builtin_amdgcn_sched_barrier(0);
         const f32x16 dp = chunks.product(v_of(stage), sub, dreg);
 #pragma unroll
@@ -709,11 +752,7 @@ __global__ __launch_bounds__(256) void attention_dq_sum_kernel(DqSumArgs a) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// dK, dV (and the dQ partial sums) of head dims 32 and 64. Every length takes
-// the split: the forward's statistics come from split scores, and scores formed
-// another way here lose their agreement with them (8 heads x 64 x 64: dQ 3.6e-7
-// against 64 bits with an fp32 kernel after the split forward, 2.5e-7 with this
-// one).
+// dK, dV (and the dQ partial sums) of head dims 32 and 64.
 template <int H, bool DQ>
 hipError_t launch_key_grad(const KeyGradArgs& a, int64_t key_blocks, hipStream_t stream) {
     hipLaunchKernelGGL((attention_key_grad_split_kernel<H, DQ>), dim3(unsigned(a.heads * key_blocks)),

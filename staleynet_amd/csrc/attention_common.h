@@ -11,6 +11,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "split_bf16.h"
+
 namespace sn {
 namespace attn {
 
@@ -69,6 +71,65 @@ struct Geometry {
     static_assert(H == 32 || H == 64 || H == 128, "head dims 32, 64, 128");
     static_assert(STAGE_SLOTS % (64 * kWaves) == 0, "whole load instructions per wave");
 };
+
+// The scores of 32 rows and 32 columns, a lane's eight h 16 c + 8 half + 0..7 of
+// its row and column from rows(c, x) and columns(c, x): split where the split
+// holds all 64 vectors and the scores come out finite, else with the fp32
+// instruction. One rule, by blocks of 32 queries and 32 keys, and one order of
+// the terms (K's part in the left factor's place: KEYS_LEFT where the rows are
+// keys) for the forward and the backward, so that the backward's scores have
+// the bits the row statistics were formed from: formed any other way they
+// differ by 2^-24 of the sums of magnitudes behind them (P off by 1e-4 at
+// scores of a few hundred).
+template <int H, bool KEYS_LEFT, int UNROLL, class Rows, class Columns>
+__device__ __forceinline__ f32x16 block_scores(Rows&& rows, Columns&& columns, bool outside, uint32_t upper) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    float least = 1.f;
+#pragma unroll UNROLL
+    for (int c = 0; c < H / 16; ++c) {
+        float x[8], y[8];
+        rows(c, x);
+        columns(c, y);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) least = fminf(least, fabsf(x[s]));
+        const SplitVector left = split_vector(x, upper), right = split_vector(y, upper);
+#pragma unroll
+        for (int t = 0; t < kTerms; ++t)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(left.part[KEYS_LEFT ? term_left(t) : term_right(t)],
+                                                          right.part[KEYS_LEFT ? term_right(t) : term_left(t)], acc, 0,
+                                                          0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // `outside`: whether this lane's column is not what the split holds.
+#pragma unroll
+    for (int r = 0; r < 16; ++r) outside |= !(fabsf(acc[r]) < INFINITY);
+    if (__any(least < kSplitLeast)) {  // or zeros
+#pragma unroll UNROLL
+        for (int c = 0; c < H / 16; ++c) {
+            float x[8];
+            rows(c, x);
+            outside |= out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+                for (int s = 0; s < 8; s += 2) f(x[s], x[s + 1]);
+            });
+        }
+    }
+    if (__any(outside)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll UNROLL
+        for (int c = 0; c < H / 16; ++c) {
+            float x[8], y[8];
+            rows(c, x);
+            columns(c, y);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
+        }
+    }
+    return acc;
+}
 
 }  // namespace attn
 }  // namespace sn

@@ -38,8 +38,8 @@
 //  * Operands outside the split's range (split_bf16.h): each thread looks at the
 //    K and V it splits, and a wave at its Q. A wave with such a value among its
 //    operands, with an output or sum that is not finite or with no finite
-//    score recomputes its queries with the fp32 instruction straight from
-//    memory. The softmax's own e^(x - m) need no look: the exponential unit
+//    score recomputes its queries straight from memory, P V and the scores of
+//    the blocks that need it (block_scores) with the fp32 instruction. The softmax's own e^(x - m) need no look: the exponential unit
 //    gives 0 under 2^-126 (as it did before the split), and the split is off by
 //    2^-134 at most on the ones between that and 2^-110, against sums of 1 or
 //    more. (The look costs 0.4 us of a prompt chunk's 20, and half a percent of
@@ -396,22 +396,16 @@ void causal_attention_kernel(AttentionArgs args) {
         lds_barrier();
     }
 
-    // The fp32 instruction, from memory, for operands the split does not hold.
-    auto scores_f32 = [&](int64_t sub0) __attribute__((always_inline)) {
-        f32x16 acc;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    // The scores from memory, by the split or with the fp32 instruction (block_scores).
+    auto scores_again = [&](int64_t sub0) __attribute__((always_inline)) {
         const int64_t key = sub0 + col;
         const float* krow = kh + (key < wg_keys ? key : 0) * H;
-        for (int c = 0; c < CHUNKS; ++c) {
-            float qv[8], kv8[8];
-            load_query(c, qv);
+        return block_scores<H, true, 1>(
+            [&](int c, float (&x)[8]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int s = 0; s < 8; ++s) kv8[s] = key < wg_keys ? krow[16 * c + 8 * half + s] : 0.f;
-#pragma unroll
-            for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv8[s], qv[s], acc, 0, 0, 0);
-        }
-        return acc;
+                for (int s = 0; s < 8; ++s) x[s] = key < wg_keys ? krow[16 * c + 8 * half + s] : 0.f;
+            },
+            load_query, outside, upper);
     };
     float poison = l * 0.f;
 #pragma unroll
@@ -426,7 +420,7 @@ void causal_attention_kernel(AttentionArgs args) {
     if (redo) {
         clear();
         for (int64_t sub0 = key_first; sub0 < wave_keys; sub0 += 32) {
-            const f32x16 s = scores_f32(sub0);
+            const f32x16 s = scores_again(sub0);
             float x[16];
             softmax(Masked{}, s, sub0, x);
 #pragma unroll
@@ -496,7 +490,7 @@ void causal_attention_kernel(AttentionArgs args) {
             if (sub0 >= args.keys) continue;
             f32x16 acc;
             if (sub0 < wave_keys) {
-                acc = redo ? scores_f32(sub0) : scores(sub);
+                acc = redo ? scores_again(sub0) : scores(sub);
             } else {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[r] = 0.f;

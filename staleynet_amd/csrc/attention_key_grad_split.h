@@ -31,7 +31,7 @@
 //    dS is one the split holds. A block with an operand outside the range, or
 //    with a sum that is not finite, is computed again by the same workgroup
 //    with the fp32 instruction from memory. (A backward whose every block is:
-//    192 heads x 1024 x 64 557 -> 1870 us. Peaked scores and gradients of a mean
+//    192 heads x 1024 x 64 557 -> 2070 us. Peaked scores and gradients of a mean
 //    loss stay at 575. A launch of their own for such blocks cost every backward
 //    2 to 9 us.)
 #pragma once
@@ -236,7 +236,9 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
 
     // The stage's 32 queries (octets of h at `rows`) against this wave's keys,
     // whose chunk c right(c, part) gives. Each chunk's fragments are read under
-    // the MFMAs of the chunk before (all at once they would spill).
+    // the MFMAs of the chunk before (all at once they would spill). The right
+    // factor's parts come first in the terms, as K's do in the forward, so that
+    // S has the bits its row statistics were formed from.
     const int row_read = (half * S::ROW_PLANE + col) * 16;
     auto product = [&](const char* rows, auto right) __attribute__((always_inline)) {
         f32x16 acc;
@@ -258,7 +260,7 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int t = 0; t < kTerms; ++t)
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[c % 2][term_left(t)], g[c % 2][term_right(t)], acc, 0,
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[c % 2][term_right(t)], g[c % 2][term_left(t)], acc, 0,
                                                               0, 0);
         }
         return acc;
@@ -495,30 +497,44 @@ void attention_key_grad_split_kernel(KeyGradArgs a) {
         return;
     }
 
-    // The block again with the fp32 instruction, operands from memory: S and dP a 32 x 32 block per wave as above, P
-    // and dS as they are, dS through LDS for dQ. Rare, and written for few registers.
+    // The block again, operands from memory: a 32 x 32 block of S (block_scores) and dP per wave as above, P and dS as
+    // they are, dS through LDS for dQ; the products with the fp32 instruction. Rare, and written for few registers.
     clear();
+    bool k_outside = false;  // this lane's K is not what the split holds
+#pragma unroll 1
+    for (int c = 0; c < CHUNKS; ++c) {
+        const float* from = a.k + head * a.kv_stride + (key_ok ? key : 0) * H + 8 * half + 16 * c;
+        k_outside |= out_of_range([&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) f(key_ok ? from[i] : 0.f, key_ok ? from[i + 1] : 0.f);
+        });
+    }
 #pragma unroll 1
     for (int64_t q0 = q_begin; q0 < a.queries; q0 += kSplitQueries) {
-        f32x16 s, dp;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            s[r] = 0.f;
-            dp[r] = 0.f;
-        }
         const float* q_head = a.q + head * a.q_stride;
         const float* d_head = a.d_out + head * a.q_stride;
         const bool row_ok = q0 + col < a.queries;
         const int64_t row = (row_ok ? q0 + col : 0) * H + 8 * half;
         const int64_t kv_row = head * a.kv_stride + (key_ok ? key : 0) * H + 8 * half;
+        const f32x16 s = block_scores<H, false, 1>(
+            [&](int c, float (&x)[8]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = row_ok ? q_head[row + 16 * c + i] : 0.f;
+            },
+            [&](int c, float (&y)[8]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = key_ok ? a.k[kv_row + 16 * c + i] : 0.f;
+            },
+            k_outside, upper);
+        f32x16 dp;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = 0.f;
 #pragma unroll 1
         for (int c = 0; c < CHUNKS; ++c) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float qv = q_head[row + 16 * c + i], dv_ = d_head[row + 16 * c + i];
-                const float kv = a.k[kv_row + 16 * c + i], vv = a.v[kv_row + 16 * c + i];
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(row_ok ? qv : 0.f, key_ok ? kv : 0.f, s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x2f32(row_ok ? dv_ : 0.f, key_ok ? vv : 0.f, dp, 0, 0, 0);
+                const float x = d_head[row + 16 * c + i], y = a.v[kv_row + 16 * c + i];
+                dp = __builtin_amdgcn_mfma_f32_32x32x2f32(row_ok ? x : 0.f, key_ok ? y : 0.f, dp, 0, 0, 0);
             }
         }
         float* ds_lds = reinterpret_cast<float*>(stage) + (32 * wave + col) * S::DS_ROW;
