@@ -18,8 +18,8 @@ BUILD_DIR = os.path.join(PACKAGE_DIR, "_build")
 LIBRARY = os.path.join(PACKAGE_DIR, "libstaleynet_gemm.so")
 INCLUDE = os.path.join(REPO_ROOT, "include")
 
-SOURCES = ["context.cpp", "gemm_f32.hip", "gemm_f32_unaligned.hip", "gemm_dma.hip", "gemm_bf16.hip", "gemm_simple.hip", "gemv.hip", "bias.hip",
-           "softmax.hip", "loss.hip", "heads.hip", "attention.hip", "attention_forward.hip", "bf16_stage.hip",
+SOURCES = ["context.cpp", "gemm_f32.hip", "gemm_f32_unaligned.hip", "gemm_dma.hip", "gemm_bf16.hip",
+           "gemm_simple.hip", "gemv.hip", "bias.hip", "softmax.hip", "loss.hip", "heads.hip", "attention.hip", "attention_forward.hip", "bf16_stage.hip",
            "synth.hip", "route.hip", "noalloc.hip", "attention_backward.hip",
            "gemm_bf16_wide.hip"]
 

@@ -18,7 +18,6 @@ namespace sn {
 namespace gemm {
 namespace {
 
-
 template <class T, class LA, class LB>
 __device__ __forceinline__ void multiply_tile_bf16(const uint16_t* __restrict__ lds_a,
                                                    const uint16_t* __restrict__ lds_b, f32x16 (&acc)[T::FM][T::FN],

@@ -30,9 +30,7 @@ namespace sn {
 namespace gemm {
 namespace {
 
-
 using WideTile = Tile<256, 256, 32, 4, 2>;
-
 
 template <int PENDING>
 __device__ __forceinline__ void wait_vector_loads() {

@@ -44,7 +44,8 @@
 //    305-312 TFLOP/s (the clock falls from 2.38 to 1.75 GHz; zeros run at
 //    2.37), 269-276 with the conversions, 234-241 with the LDS traffic and
 //    216-226 with the operand loads besides. The large layer's products run
-//    at 170-200 (the fp32 instruction: 136-140), so less work beside the
+//    at 170-190 (the fp32 instruction: 136-140) with the matrix cores busy 58
+//    to 60 % of the cycles at 1.65 GHz, so less work beside the
 //    MFMAs is what would make it faster; deeper prefetch and other issue
 //    orders changed cycles and clock by the same factor.
 //
@@ -70,7 +71,8 @@
 // lane half h of chunk c reads octet 2 c + h). Writes are 8 bytes (four k):
 // the four-slot pad puts the octets of a 16-lane write phase 64 bytes apart,
 // so 8 k-groups x 2 rows (K-contiguous) or 2 groups x 8 row blocks
-// (row-contiguous) fall on distinct banks. Where a wave has two blocks on a
+// (row-contiguous) fall on distinct banks of that phase (counted over all LDS
+// instructions, two conflict cycles each remain). Where a wave has two blocks on a
 // side their rows interleave (block i's position q holds row 2 q + i of the
 // wave's 64): a row-contiguous loader's block of four rows then writes
 // slots two apart, and a lane's two columns are adjacent in the output (one

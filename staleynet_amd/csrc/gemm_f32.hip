@@ -184,7 +184,6 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const f32x4* __rest
     }
 }
 
-
 // The split-K model's view of a tile: workgroups per CU, and the rate one CU
 // sustains on it.
 template <class T>
@@ -200,23 +199,23 @@ Plan f32_plan(const Problem& p, const Env& env) {
 }
 
 // Products whose 128x128 plan (split K included) has fewer workgroups than
-// the device has CUs take 64x64 tiles (four waves of 32x32, five workgroups
-// per CU by LDS): the 7.1M model's products and the reference's published shapes
-// (2048 x 768 x 256: 96 tiles of 128 x 128 on 256 CUs). Measured: the 7.1M model's
-// set 43.6 -> 56.1 TFLOP/s, 2048 x 768 x 256 34 -> 54, 2048 x 1024 x 256
-// 45 -> 68; the 42.9M and 111.5M models, whose plans fill the CUs, keep 128 x 128 (a
-// 128 x 64 tile below 256 tiles lost 6 % on the 111.5M model's 768 x 768 weight
-// gradient).
+// the device has CUs take 64x64 tiles (four waves of 32x32, four workgroups
+// per CU): the 7.1M model's products and the reference's published shapes
+// (2048 x 768 x 256: 96 tiles of 128 x 128 on 256 CUs). Measured, 64x64 against
+// 128x128: NN 2048 x 768 x 256 12.8 against 17.0 us, 2048 x 1024 x 256 12.7
+// against 17.3, 2048 x 256 x 1024 19.0 against 23.6, TN 256 x 1024 x 2048 19.8
+// against 23.0; the 42.9M and 111.5M models, whose plans fill the CUs, keep
+// 128 x 128.
 // Products whose 128x128 plan leaves CU slots empty (under two workgroups
-// per CU) with under 24 K-steps per workgroup take 64x64 tiles as well: the
-// 128x128 plan there splits an already short K (or runs one workgroup per
-// CU), and each workgroup's start-up and epilogue weigh on a few K-steps;
-// four 64x64 workgroups per CU fill the device without splitting. Measured
-// (fp32, one GPU's share of config 2 over 8 GPUs, M = 4096): NN and NT
-// 4096 x 768 x 768 74-76 -> 104-107 TFLOP/s, TN 768 x 768 x 4096 83 -> 89;
-// the 42.9M model's NN and NT 8192 x 512 x 512 99-103 -> 102-105. Longer
-// slices keep 128x128 (the 111.5M model's 768 x 768 x 32768 weight
-// gradient, 74 K-steps a workgroup: 127 TFLOP/s against 119 on 64x64).
+// per CU) with under 24 K-steps per workgroup take 64x64 tiles as well: four
+// 64x64 workgroups per CU fill the device without splitting a short K. The line
+// was drawn with the fp32 matrix instruction, whose K-steps were 2.7 times as
+// long, and holds for some of these only: NN and NT 4096 x 768 x 768 (one GPU's
+// share of the 111.5M set over 8) 39.1 and 36.9 us against 43.1 and 42.5, but
+// TN 768 x 768 x 4096 50.7 against 39.6 and NN 8192 x 512 x 512 34.4 against
+// 30.4, where 128x128 tiles are the better ones now. Longer slices keep
+// 128x128 (the 111.5M model's 768 x 768 x 32768 weight gradient, 74 K-steps a
+// workgroup: 205 us against 318 on 64x64).
 constexpr int64_t kSmallTileMaxK = 768;
 
 // Whether 16-byte loads serve both operands of `p` on tile T.
